@@ -238,6 +238,8 @@ struct GemmArgs {             // MFMA GEMM (gemm.hip): out = epi(x . w^T), x [M,
   int csw;
   int cph;
   int cpw;
+  int gn;                     // tile.hip: column tiles per group of the tile order (>= 1)
+  int gpad;
 };
 
 struct ConvArgs {             // implicit-GEMM conv2d (conv.hip), NCHW activations, OIHW weights, groups 1
@@ -938,5 +940,79 @@ __device__ __forceinline__ float block_max256(float v, float* red) {
   if (l == 0) red[w] = v;
   __syncthreads();
   return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+#endif
+
+#if defined(__HIPCC__) && !defined(__HIPCC_RTC__)
+// ---------------------------------------------------------------- MFMA GEMM helpers (gemm.hip, tile.hip)
+
+enum { GE_BIAS = 0, GE_RESID = 1, GE_SILU = 2, GE_CONV = 3 };
+
+template <int DT>
+__device__ __forceinline__ float gm_ld(const void* p, long long i) {
+  const uint16_t h = ((const uint16_t*)p)[i];
+  return DT == HS_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
+}
+
+template <int DT>
+__device__ __forceinline__ float gm_round(float f) {
+  return DT == HS_BF16 ? bf16_to_f32(f32_to_bf16(f)) : f16_to_f32(f32_to_f16(f));
+}
+
+template <int DT>
+__device__ __forceinline__ uint16_t gm_pack(float f) {
+  return DT == HS_BF16 ? f32_to_bf16(f) : f32_to_f16(f);
+}
+
+// two values rounded to DT, the first in the low half
+template <int DT>
+__device__ __forceinline__ uint32_t gm_pack2(float lo, float hi) {
+  if constexpr (DT == HS_BF16) {
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 b16x2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), b16x2));
+  } else {
+    return (uint32_t)f32_to_f16(lo) | ((uint32_t)f32_to_f16(hi) << 16);
+  }
+}
+template <int DT>
+__device__ __forceinline__ float gm_lo(uint32_t w) {
+  return DT == HS_BF16 ? __uint_as_float(w << 16) : f16_to_f32((uint16_t)(w & 0xffffu));
+}
+template <int DT>
+__device__ __forceinline__ float gm_hi(uint32_t w) {
+  return DT == HS_BF16 ? __uint_as_float(w & 0xffff0000u) : f16_to_f32((uint16_t)(w >> 16));
+}
+
+// v / (1 + e^-v) of a value already rounded to 16 bits, in 10 instructions (the library's expf and
+// an IEEE division take about 25, and an epilogue is 10 us of a 1000 x 8960 output's 53): both
+// sides of the fraction scaled by 1/4 so that the reciprocal stays a normal number down to v = -88.7
+// (where expf overflows), one remainder step on the quotient (skipped where the remainder is zero or
+// NaN: v = -0, and the infinities). Over all 2^16 inputs its rounding to 16 bits differs from the
+// correctly rounded result as often as the library form's does: 17 times in bfloat16, once in float16.
+__device__ __forceinline__ float gm_silu(float v) {
+  const float d = 0.25f + __builtin_amdgcn_exp2f(__builtin_fmaf(v, -1.44269504088896340736f, -2.f));
+  const float v4 = 0.25f * v, r = __builtin_amdgcn_rcpf(d), q = v4 * r, rem = __builtin_fmaf(-q, d, v4);
+  return (rem < 0.f || rem > 0.f) ? __builtin_fmaf(rem, r, q) : q;
+}
+
+// s_waitcnt vmcnt(N), the other counters untouched
+template <int N>
+__device__ __forceinline__ void gm_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (7 << 4) | (0xF << 8));
+}
+// wait until at most `after` stages of NI loads each are outstanding (after <= MAXA, uniform)
+template <int NI, int MAXA>
+__device__ __forceinline__ void gm_vmcnt_after(int after) {
+  if constexpr (MAXA > 0) {
+    if (after >= MAXA) {
+      gm_vmcnt<MAXA * NI>();
+      return;
+    }
+    gm_vmcnt_after<NI, MAXA - 1>(after);
+  } else {
+    gm_vmcnt<0>();
+  }
 }
 #endif

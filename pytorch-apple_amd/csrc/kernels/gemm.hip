@@ -1,4 +1,6 @@
-// MFMA GEMM for prefill-shaped linears (M >= 64): out[m, n] = epi(sum_k x[m, k] w[n, k]).
+// MFMA GEMM on 4-wave workgroups: out[m, n] = epi(sum_k x[m, k] w[n, k]). The linears with
+// K % 64 == 0 run on tile.hip; here are the others (K % 32 == 0), the batched matmuls, the
+// convolutions and the split-K reduces of both.
 //
 // Both operands are K-contiguous ([M, K] activations, [N, K] weights as the model stores
 // them), which is exactly the register layout of the gfx950 MFMA
@@ -6,7 +8,7 @@
 // at k offset 8 * (l / 32), and the 32x32 fp32 result sits in 16 registers per lane,
 // element 4q + r at row 8q + 4(l / 32) + r, column l % 32.
 // Workgroup tile BM x BN (BN columns per weight), K step 32, 256 threads as 2 x 2
-// waves of (BM / 2) x (BN / 2) (or 4 x 1 waves: GEMM_KERNEL_W4). Tiles are double-buffered in LDS through registers: the
+// waves of (BM / 2) x (BN / 2). Tiles are double-buffered in LDS through registers: the
 // global loads of step k+1 are in flight while step k is multiplied, then stored to the
 // other buffer, one barrier per step. LDS rows are padded (40 elements) so the 16-byte
 // fragment reads of 32 consecutive rows spread over the banks.
@@ -26,7 +28,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 gm_bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 gm_f16x8;
 typedef __attribute__((ext_vector_type(16))) float gm_f32x16;
 
-enum { GE_BIAS = 0, GE_RESID = 1, GE_SILU = 2, GE_CONV = 3 };
 #define GM_BK 32      // default K step
 
 template <int DT>
@@ -37,22 +38,6 @@ __device__ __forceinline__ gm_f32x16 gm_mfma(const uint4 a, const uint4 b, gm_f3
   else
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(gm_f16x8, a), __builtin_bit_cast(gm_f16x8, b),
                                                   c, 0, 0, 0);
-}
-
-template <int DT>
-__device__ __forceinline__ float gm_ld(const void* p, long long i) {
-  const uint16_t h = ((const uint16_t*)p)[i];
-  return DT == HS_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
-}
-
-template <int DT>
-__device__ __forceinline__ float gm_round(float f) {
-  return DT == HS_BF16 ? bf16_to_f32(f32_to_bf16(f)) : f16_to_f32(f32_to_f16(f));
-}
-
-template <int DT>
-__device__ __forceinline__ uint16_t gm_pack(float f) {
-  return DT == HS_BF16 ? f32_to_bf16(f) : f32_to_f16(f);
 }
 
 // slot permutation of the direct-to-LDS rows (GM_SWZ_PAIR: rows 2j and 2j + 1 share one,
@@ -69,26 +54,6 @@ __device__ __forceinline__ int gm_swz(int r) { return GM_SWZ_PAIR ? (r >> 1) & 7
 __device__ __forceinline__ void gm_dma16(const void* g, unsigned lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
 }
-// s_waitcnt vmcnt(N), the other counters untouched
-template <int N>
-__device__ __forceinline__ void gm_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (7 << 4) | (0xF << 8));
-}
-// wait until at most `after` stages of NI loads each are outstanding (after <= MAXA, uniform)
-template <int NI, int MAXA>
-__device__ __forceinline__ void gm_vmcnt_after(int after) {
-  if constexpr (MAXA > 0) {
-    if (after >= MAXA) {
-      gm_vmcnt<MAXA * NI>();
-      return;
-    }
-    gm_vmcnt_after<NI, MAXA - 1>(after);
-  } else {
-    gm_vmcnt<0>();
-  }
-}
-
 // conv epilogue (conv.hip's rounding points): after v = round(acc + bias),
 //   batch norm: v = round(v * al + be), al = w / sqrt(var + eps), be = bias - mean * al;
 //   residual: v = round(v + r);  ReLU: v = max(v, 0) (NaN kept)
@@ -108,7 +73,7 @@ __device__ __forceinline__ float gm_conv_tail(const GemmArgs& a, float v, float 
 }
 
 // STAGES 0: LDS double buffer filled through registers (the loads of step s + 1 are in flight
-// while step s is multiplied). STAGES >= 2 (BK 64, not KN): the operands go from global memory
+// while step s is multiplied). STAGES >= 2 (the convolutions; BK 64): the operands go from global memory
 // straight into LDS (gfx950 global_load_lds_dwordx4), STAGES buffers deep, so the loads of
 // steps s + 1 .. s + STAGES - 1 are in flight while step s is multiplied and no registers hold
 // them. Those rows are unpadded 128-byte rows; 16-byte chunk c of row r sits in slot
@@ -117,7 +82,7 @@ __device__ __forceinline__ float gm_conv_tail(const GemmArgs& a, float v, float 
 // 1: k = (kh, kw, ci), a whole 64-channel block per K step, padded taps read a.zero;
 // 2: a zero-bordered 4-channel image, each 16-byte chunk two neighbouring taps of one kernel row.
 template <int DT, int EPI, int NW, int BM, int BN, bool KN = false, int BK = GM_BK, bool GRP = false,
-          int STAGES = 0, int CV = 0, int WR = 2, int LDSST = 0>
+          int STAGES = 0, int CV = 0, int LDSST = 0>
 __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
   constexpr bool DMA = STAGES >= 2;
   // LDSST 1 (direct-to-LDS): the LDS of one stage, each K step loaded and waited for in turn (other
@@ -125,13 +90,13 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
   constexpr int LST = LDSST > 0 ? LDSST : STAGES;
   static_assert(LDSST == 0 || (DMA && LDSST == 1), "LDS stages");
   static_assert(!DMA || (BK == 64 && !KN), "direct-to-LDS staging: BK 64, K-contiguous weights");
-  static_assert(!CV || (DMA && NW == 1 && !GRP), "conv gather: direct-to-LDS, one weight");
+  static_assert(!DMA || (NW == 1 && !GRP), "direct-to-LDS staging: the convolutions");
+  static_assert(!CV || DMA, "conv gather: direct-to-LDS");
   constexpr int LDK = BK + 8;             // padded LDS row (elements): fragment reads of 32 rows spread over the banks
   constexpr int CPR = BK / 8;             // 16-byte chunks per staged row
   constexpr int BNT = BN * NW;            // weight rows staged per step (BN columns per weight)
-  // the 4 waves as WR rows x WC columns of (BM / WR) x (BN / WC) each (per weight)
-  static_assert(WR == 1 || WR == 2 || WR == 4, "wave rows");
-  constexpr int WC = 4 / WR, WM = BM / WR, WN = BN / WC;
+  // the 4 waves as 2 rows x 2 columns of (BM / 2) x (BN / 2) each (per weight)
+  constexpr int WC = 2, WM = BM / 2, WN = BN / 2;
   static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile");
   constexpr int TI = WM / 32;             // 32-row MFMA tiles per wave
   constexpr int TJ = WN / 32;             // 32-column MFMA tiles per wave and weight
@@ -395,13 +360,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       const int row = (wave * NB + q) * 8 + lr;
-      const uint16_t* wrow;
-      if constexpr (GRP) {
-        wrow = W0 + (long long)(min(n_base + row, g_hi - 1) - g_lo) * a.ldw;
-      } else {
-        const int u = row / BN, n = min(n_base + row % BN, a.N - 1);
-        wrow = (u == 0 ? W0 : W1) + (long long)n * a.ldw;
-      }
+      const uint16_t* wrow = W0 + (long long)min(n_base + row, a.N - 1) * a.ldw;
       bsrc[q] = (const char*)wrow + ((ls ^ gm_swz(row)) * 16);
     }
     auto issue = [&](int st) {   // stage st of the K loop into LDS buffer st % LST
@@ -756,64 +715,38 @@ extern "C" __global__ void __launch_bounds__(256) k_gemm_reduce_f16_resid_norm(c
 // up to 2 waves per SIMD: the 64 accumulator registers plus staging and fragments need
 // more than the default register budget, which would otherwise spill the staging to scratch
 #define GM_ATTRS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
-// Each kernel comes in two K steps: 32, and 64 (suffix _k64: twice the MFMA work per barrier and
-// per prefetch, which hides the operand latency better; 73.7 KB of LDS for 128 x 128 tiles, so two
-// workgroups still share a CU). Measured at M = 512, K = 1536: lm_head 381 -> 312 us, gate/up
-// 61 -> 51 us; K = 8960 down 39 -> 30 us. The host takes _k64 when K (and the split-K chunk) is a
-// multiple of 64. Suffix _k64d: K step 64 with direct-to-LDS staging, ST buffers deep (the stage
-// count fits two workgroups per CU where the tile allows). Measured at M = 512 (same launch,
-// bit-identical results): gate/up 64 x 64 57 -> 52 us, down 128 x 128 with 4 K splits 31 -> 26 us,
-// o_proj 64 x 64 with 2 K splits 15.8 -> 9.5 us, q | k | v 14.6 -> 11.4 us; the lm_head's 4,748
-// tiles of 128 x 128 keep enough workgroups in flight without it (324 us against 367).
-#define GEMM_KERNEL(NAME, DT, EPI, NW, BM, BN, ST)                                                      \
-  extern "C" __global__ void GM_ATTRS NAME(const GemmArgs a) { gemm_body<DT, EPI, NW, BM, BN>(a); }     \
-  extern "C" __global__ void GM_ATTRS NAME##_k64(const GemmArgs a) { gemm_body<DT, EPI, NW, BM, BN, false, 64>(a); } \
-  extern "C" __global__ void GM_ATTRS NAME##_k64d(const GemmArgs a) {                                  \
-    gemm_body<DT, EPI, NW, BM, BN, false, 64, false, ST>(a);                                           \
-  }
+// K step 32; the batched matmuls also come with 64 (suffix _k64: twice the MFMA work per barrier and
+// per prefetch). Linears with K % 64 == 0 run on tile.hip.
+#define GEMM_KERNEL(NAME, DT, EPI, NW, BM, BN)                                                          \
+  extern "C" __global__ void GM_ATTRS NAME(const GemmArgs a) { gemm_body<DT, EPI, NW, BM, BN>(a); }
+#define GEMM_KERNEL_K64(NAME, DT, EPI, NW, BM, BN)                                                      \
+  extern "C" __global__ void GM_ATTRS NAME##_k64(const GemmArgs a) { gemm_body<DT, EPI, NW, BM, BN, false, 64>(a); }
 #define GEMM_KERNEL_KN(NAME, DT, BM, BN)                                                                  \
   extern "C" __global__ void GM_ATTRS NAME(const GemmArgs a) { gemm_body<DT, GE_BIAS, 1, BM, BN, true>(a); } \
   extern "C" __global__ void GM_ATTRS NAME##_k64(const GemmArgs a) { gemm_body<DT, GE_BIAS, 1, BM, BN, true, 64>(a); }
 #define GEMM_REDUCE(NAME, DT, EPI) \
   extern "C" __global__ void __launch_bounds__(256) NAME(const GemmArgs a) { gemm_reduce_body<DT, EPI>(a); }
 
-// k_gemm_<dtype>_<epilogue>_m<BM>n<BN>: BN columns per weight; last argument: direct-to-LDS stages
-GEMM_KERNEL(k_gemm_bf16_bias_m128n128, HS_BF16, GE_BIAS, 1, 128, 128, 4)
-GEMM_KERNEL(k_gemm_bf16_bias_m64n128, HS_BF16, GE_BIAS, 1, 64, 128, 3)
-GEMM_KERNEL(k_gemm_bf16_bias_m64n64, HS_BF16, GE_BIAS, 1, 64, 64, 4)
-GEMM_KERNEL(k_gemm_bf16_resid_m128n128, HS_BF16, GE_RESID, 1, 128, 128, 4)
-GEMM_KERNEL(k_gemm_bf16_resid_m64n128, HS_BF16, GE_RESID, 1, 64, 128, 3)
-GEMM_KERNEL(k_gemm_bf16_resid_m64n64, HS_BF16, GE_RESID, 1, 64, 64, 4)
-GEMM_KERNEL(k_gemm_bf16_silu_m128n64, HS_BF16, GE_SILU, 2, 128, 64, 3)
-GEMM_KERNEL(k_gemm_bf16_silu_m64n64, HS_BF16, GE_SILU, 2, 64, 64, 3)
-GEMM_KERNEL(k_gemm_f16_bias_m128n128, HS_F16, GE_BIAS, 1, 128, 128, 4)
-GEMM_KERNEL(k_gemm_f16_bias_m64n128, HS_F16, GE_BIAS, 1, 64, 128, 3)
-GEMM_KERNEL(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64, 4)
-GEMM_KERNEL(k_gemm_f16_resid_m128n128, HS_F16, GE_RESID, 1, 128, 128, 4)
-GEMM_KERNEL(k_gemm_f16_resid_m64n128, HS_F16, GE_RESID, 1, 64, 128, 3)
-GEMM_KERNEL(k_gemm_f16_resid_m64n64, HS_F16, GE_RESID, 1, 64, 64, 4)
-// direct-to-LDS only, the 4 waves as 4 rows x 1 column (wave tile BM / 4 x BN per weight): for tile
-// widths that are an odd multiple of 32 (BN = 96: 94 column tiles of a 8960-row weight pair, so
-// M = 512 takes 376 workgroups, one round at two per CU; a 1536-row weight over K = 8960, 64
-// tiles x 8 K splits, one round of 512)
-#define GEMM_KERNEL_W4(NAME, DT, EPI, NW, BM, BN, ST)                                                   \
-  extern "C" __global__ void GM_ATTRS NAME##_k64d(const GemmArgs a) {                                  \
-    gemm_body<DT, EPI, NW, BM, BN, false, 64, false, ST, 0, 4>(a);                                     \
-  }
-GEMM_KERNEL_W4(k_gemm_bf16_silu_m128n96, HS_BF16, GE_SILU, 2, 128, 96, 2)
-GEMM_KERNEL_W4(k_gemm_f16_silu_m128n96, HS_F16, GE_SILU, 2, 128, 96, 2)
-GEMM_KERNEL_W4(k_gemm_bf16_resid_m128n96, HS_BF16, GE_RESID, 1, 128, 96, 2)
-GEMM_KERNEL_W4(k_gemm_f16_resid_m128n96, HS_F16, GE_RESID, 1, 128, 96, 2)
-GEMM_KERNEL_W4(k_gemm_bf16_bias_m128n96, HS_BF16, GE_BIAS, 1, 128, 96, 2)
-GEMM_KERNEL_W4(k_gemm_f16_bias_m128n96, HS_F16, GE_BIAS, 1, 128, 96, 2)
+// k_gemm_<dtype>_<epilogue>_m<BM>n<BN>: BN columns per weight
+GEMM_KERNEL(k_gemm_bf16_bias_m128n128, HS_BF16, GE_BIAS, 1, 128, 128)
+GEMM_KERNEL(k_gemm_bf16_bias_m64n128, HS_BF16, GE_BIAS, 1, 64, 128)
+GEMM_KERNEL(k_gemm_bf16_bias_m64n64, HS_BF16, GE_BIAS, 1, 64, 64)
+GEMM_KERNEL(k_gemm_bf16_resid_m128n128, HS_BF16, GE_RESID, 1, 128, 128)
+GEMM_KERNEL(k_gemm_bf16_resid_m64n128, HS_BF16, GE_RESID, 1, 64, 128)
+GEMM_KERNEL(k_gemm_bf16_resid_m64n64, HS_BF16, GE_RESID, 1, 64, 64)
+GEMM_KERNEL(k_gemm_bf16_silu_m128n64, HS_BF16, GE_SILU, 2, 128, 64)
+GEMM_KERNEL(k_gemm_bf16_silu_m64n64, HS_BF16, GE_SILU, 2, 64, 64)
+GEMM_KERNEL(k_gemm_f16_bias_m128n128, HS_F16, GE_BIAS, 1, 128, 128)
+GEMM_KERNEL(k_gemm_f16_bias_m64n128, HS_F16, GE_BIAS, 1, 64, 128)
+GEMM_KERNEL(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64)
+GEMM_KERNEL_K64(k_gemm_bf16_bias_m128n128, HS_BF16, GE_BIAS, 1, 128, 128)
+GEMM_KERNEL_K64(k_gemm_bf16_bias_m64n64, HS_BF16, GE_BIAS, 1, 64, 64)
+GEMM_KERNEL_K64(k_gemm_f16_bias_m128n128, HS_F16, GE_BIAS, 1, 128, 128)
+GEMM_KERNEL_K64(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64)
 
 // grouped (q | k | v projections of one activation into one [M, N] output; no split K)
-#define GEMM_KERNEL_GRP(NAME, DT, BM, BN, ST)                                                                  \
-  extern "C" __global__ void GM_ATTRS NAME(const GemmArgs a) { gemm_body<DT, GE_BIAS, 1, BM, BN, false, 32, true>(a); } \
-  extern "C" __global__ void GM_ATTRS NAME##_k64(const GemmArgs a) { gemm_body<DT, GE_BIAS, 1, BM, BN, false, 64, true>(a); } \
-  extern "C" __global__ void GM_ATTRS NAME##_k64d(const GemmArgs a) {                                              \
-    gemm_body<DT, GE_BIAS, 1, BM, BN, false, 64, true, ST>(a);                                                     \
-  }
+#define GEMM_KERNEL_GRP(NAME, DT, BM, BN)                                                                      \
+  extern "C" __global__ void GM_ATTRS NAME(const GemmArgs a) { gemm_body<DT, GE_BIAS, 1, BM, BN, false, 32, true>(a); }
 // conv2d on channels-last activations (conv epilogue): _conv takes x as the [pixels, Cin] rows of
 // an NHWC image (1 x 1, stride 1, no padding); _convg gathers the taps of any kernel / stride /
 // padding (Cin % 64 == 0) with direct-to-LDS staging; _convp reads a zero-bordered 4-channel image
@@ -849,10 +782,10 @@ GEMM_KERNEL_W4(k_gemm_f16_bias_m128n96, HS_F16, GE_BIAS, 1, 128, 96, 2)
 // short K (1 x 1 convs over few channels): the LDS of one stage, 16 KB at 64 x 64, so up to eight
 // workgroups share a CU
 extern "C" __global__ void GM_ATTRS_CONV k_gemm_f16_conv_m64n64_k64d1(const GemmArgs a) {
-  gemm_body<HS_F16, GE_CONV, 1, 64, 64, false, 64, false, 2, 0, 2, 1>(a);
+  gemm_body<HS_F16, GE_CONV, 1, 64, 64, false, 64, false, 2, 0, 1>(a);
 }
 extern "C" __global__ void GM_ATTRS_CONV k_gemm_bf16_conv_m64n64_k64d1(const GemmArgs a) {
-  gemm_body<HS_BF16, GE_CONV, 1, 64, 64, false, 64, false, 2, 0, 2, 1>(a);
+  gemm_body<HS_BF16, GE_CONV, 1, 64, 64, false, 64, false, 2, 0, 1>(a);
 }
 GEMM_CONV(f16, HS_F16, 128, 128, 4)
 GEMM_CONV(f16, HS_F16, 128, 64, 3)
@@ -864,10 +797,8 @@ GEMM_CONV(bf16, HS_BF16, 64, 128, 3)
 GEMM_CONV(bf16, HS_BF16, 64, 64, 4)
 GEMM_REDUCE(k_gemm_reduce_f16_conv, HS_F16, GE_CONV)
 GEMM_REDUCE(k_gemm_reduce_bf16_conv, HS_BF16, GE_CONV)
-GEMM_KERNEL_GRP(k_gemm_bf16_grp_m64n64, HS_BF16, 64, 64, 4)
-GEMM_KERNEL_GRP(k_gemm_bf16_grp_m128n128, HS_BF16, 128, 128, 4)
-GEMM_KERNEL_GRP(k_gemm_f16_grp_m64n64, HS_F16, 64, 64, 4)
-GEMM_KERNEL_GRP(k_gemm_f16_grp_m128n128, HS_F16, 128, 128, 4)
+GEMM_KERNEL_GRP(k_gemm_bf16_grp_m64n64, HS_BF16, 64, 64)
+GEMM_KERNEL_GRP(k_gemm_bf16_grp_m128n128, HS_BF16, 128, 128)
 GEMM_REDUCE(k_gemm_reduce_bf16_bias, HS_BF16, GE_BIAS)
 GEMM_REDUCE(k_gemm_reduce_bf16_resid, HS_BF16, GE_RESID)
 GEMM_REDUCE(k_gemm_reduce_bf16_silu, HS_BF16, GE_SILU)

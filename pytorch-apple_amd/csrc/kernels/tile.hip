@@ -1,0 +1,301 @@
+// MFMA GEMM on wide workgroups: out[m, n] = epi(sum_k x[m, k] w[n, k]) for activations [M, K] and
+// weights [N, K] as the model stores them, K % 64 == 0. One workgroup of WR x WC waves (8 or 12) per
+// CU and BM x BN output tile.
+//
+// What bounds a GEMM of these shapes (M = 128 .. 4096 against 1536- to 151936-row weights) is how
+// many operand bytes a CU has in flight and takes in per MFMA, not the MFMA rate itself. So:
+//   * the LDS of the whole CU (up to 160 KB) holds one workgroup's ring of ST stages of 64 of K,
+//     filled by global_load_lds_dwordx4 (128-byte rows, whole cache lines; 64-byte rows, twice as
+//     many stages of half the depth, were 10-15% slower: each line is then fetched twice);
+//   * tiles are as large as the shape allows while the grid still fills the 256 CUs in whole
+//     rounds (the host's tile_plan): 256 x 144 of both SiLU weights is 252 workgroups at M = 1000;
+//   * each operand address is a scalar base plus a 32-bit lane offset (one SALU add per load);
+//   * 12 waves (three per SIMD) on the tiles whose widths are 3 x 96 or 3 x 48, 8 on the others; the
+//     16-byte chunks of a row sit in slot c ^ ((row >> 1) & 7), which the 16 x 4 fragment reads of
+//     v_mfma_f32_16x16x32 cross without a bank conflict (237 bytes per clock and CU measured; 63 with
+//     the chunks in order).
+// The MFMA computes the transposed tile (weights as operand A), so that a lane holds 4 consecutive
+// columns of one row: 8-byte LDS writes in the epilogue, 16-byte rows out of it, and float4 partials.
+//
+// Measured on MI355X (bf16, kernel alone, weights rotated through 4 copies), against the 4-wave
+// kernels of gemm.hip: gate/up with SiLU (N = 8960, K = 1536) at M = 512 / 1000 / 2000
+// 47 / 75 / 142 -> 32 / 50 / 97 us; lm_head 512 x 151936 x 1536 325 -> 234 us (1,020 TFLOP/s);
+// down_proj (N = 1536, K = 8960) at M = 512, 5 K splits, 26 -> 20 us, at 1000 60 -> 32 us plus the
+// reduce. A steady K step of 256 x 256 takes 1.56 us (1,376 TFLOP/s over 256 CUs); a launch spends
+// the rest (8-11 us) on its first stage's latency and its epilogue.
+//
+// Epilogues (fp32 accumulator, ATen's rounding points), rows past M and columns past N clamped when
+// read and not stored:
+//   BIAS  out = round(acc + b)
+//   RESID out = round(r + round(acc + b))
+//   SILU  out = round(round(silu(round(acc_g + b_g))) * round(acc_u + b_u))   (NW = 2)
+// ksplit > 1: grid.z workgroups take kchunk of K each and store fp32 partials [z, NW, M, N]; a
+// k_gemm_reduce_* kernel (gemm.hip) sums them in order and applies the epilogue.
+// GRP: output columns [0, n1), [n1, n2), [n2, N) come from three weights and biases (n1, n2
+// multiples of BN), e.g. q | k | v of one activation.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 tg_bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 tg_f16x8;
+typedef __attribute__((ext_vector_type(4))) float tg_f32x4;
+
+template <int DT>
+__device__ __forceinline__ tg_f32x4 tg_mfma(const uint4 a, const uint4 b, tg_f32x4 c) {
+  if constexpr (DT == HS_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tg_bf16x8, a), __builtin_bit_cast(tg_bf16x8, b),
+                                                   c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(tg_f16x8, a), __builtin_bit_cast(tg_f16x8, b),
+                                                  c, 0, 0, 0);
+}
+
+// 16 bytes per lane from base + off into LDS at lds + 16 * lane. Inline assembly, so that the compiler
+// does not wait for it before every LDS read; the waits are explicit (gm_vmcnt_after).
+__device__ __forceinline__ void tg_dma16(const void* base, unsigned off, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
+template <int DT, int EPI, int NW, int BM, int BN, int WR, int WC, int ST, bool GRP = false>
+__device__ __forceinline__ void tile_body(const GemmArgs& a) {
+  constexpr int NWV = WR * WC, NTH = 64 * NWV, BNT = BN * NW;
+  constexpr int WM = BM / WR, WN = BN / WC, TI = WM / 16, TJ = WN / 16;   // wave tile, in 16 x 16 MFMA tiles
+  static_assert(WM % 16 == 0 && WN % 16 == 0 && BM % 16 == 0 && BN % 16 == 0, "wave tile");
+  constexpr int RB = 128, ROWS = BM + BNT, SB = ROWS * RB;   // bytes per staged row and per stage
+  constexpr int INS = ROWS / 8, NI = (INS + NWV - 1) / NWV;  // loads (8 rows each) per stage, per wave and stage
+  constexpr int TLD = BN + 8;                                // epilogue tile row (elements)
+  static_assert(ST * SB >= BM * TLD * 2 || ST == 2, "epilogue tile");
+  constexpr int LDSB = ST * SB > BM * TLD * 2 ? ST * SB : BM * TLD * 2;
+  __shared__ __attribute__((aligned(16))) char Ls[LDSB];
+  __shared__ __attribute__((aligned(16))) float Fb[NW * BN];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WC, wc = wave % WC;
+  // XCD-aware tile order: workgroup L runs on XCD L % 8, so L is remapped to give each XCD a contiguous
+  // range of tiles, ordered in groups of gn column tiles, row tiles next, columns within the group
+  // fastest: the range is then a block of about gn columns, whose weights and activations the XCD's
+  // L2 fetches once
+  const unsigned gx = gridDim.x, gy = gridDim.y, total = gx * gy * gridDim.z;
+  const unsigned lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+  const unsigned per = (total + 7) / 8, xcd = lin % 8, loc = lin / 8;
+  const unsigned tall = total % 8 == 0 ? 8 : total % 8;   // XCDs that get `per` tiles; the rest get per - 1
+  const unsigned tile = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+  const unsigned kz = tile / (gx * gy), t2 = tile - kz * gx * gy, gn = (unsigned)max(a.gn, 1);
+  const unsigned grp0 = t2 / (gn * gy) * gn, gw = min(gn, gx - grp0), t3 = t2 - grp0 * gy;
+  const int m_base = (int)(t3 / gw) * BM, n_base = (int)(grp0 + t3 % gw) * BN;
+  const int M = (int)a.M, N = a.N;
+  const int kbeg = (int)kz * a.kchunk, nsteps = min(a.kchunk, a.K - kbeg) / 64;
+  int g_lo = 0, g_hi = N;   // GRP: the columns of this tile's group
+  const void *W0 = a.w, *B0 = a.bias;
+  if constexpr (GRP) {
+    const int g = (n_base >= a.n1) + (n_base >= a.n2);
+    g_lo = g == 0 ? 0 : (g == 1 ? a.n1 : a.n2);
+    g_hi = g == 0 ? a.n1 : (g == 1 ? a.n2 : N);
+    W0 = g == 0 ? a.w : (g == 1 ? a.w2 : a.w3);
+    B0 = g == 0 ? a.bias : (g == 1 ? a.bias2 : a.bias3);
+  }
+  // staging: load i of this wave fills rows 8q .. 8q + 7 of a stage (x rows, then each weight's); lane ->
+  // row 8q + lane / 8, slot lane % 8. The loads past INS repeat the last one (same bytes, same place)
+  unsigned voff[NI];
+  const char* gb[NI];
+  unsigned ldst[NI];
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)&Ls[0];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int q = min(wave + i * NWV, INS - 1), r = 8 * q + (lane >> 3);
+    const unsigned chunk = (unsigned)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+    ldst[i] = lds0 + (unsigned)q * 1024u;
+    if (8 * q < BM) {
+      gb[i] = (const char*)a.x + ((long long)m_base * a.ldx + kbeg) * 2;
+      voff[i] = (unsigned)(min(m_base + r, M - 1) - m_base) * (unsigned)(a.ldx * 2) + chunk;
+    } else {
+      const int u = (8 * q - BM) / BN, rr = r - BM - u * BN;
+      gb[i] = (const char*)(u == 0 ? W0 : a.w2) + ((long long)(n_base - g_lo) * a.ldw + kbeg) * 2;
+      voff[i] = (unsigned)(min(n_base + rr, g_hi - 1) - n_base) * (unsigned)(a.ldw * 2) + chunk;
+    }
+  }
+  // the tile's bias columns, loaded ahead of the operands, kept in a register until the epilogue
+  float bv[NW];
+#pragma unroll
+  for (int u = 0; u < NW; ++u) bv[u] = 0.f;
+  if (tid < BN && a.ksplit == 1) {
+    const int n = min(n_base + tid, g_hi - 1) - g_lo;
+    if (a.flags & 1) bv[0] = gm_ld<DT>(B0, n);
+    if constexpr (NW == 2)
+      if (a.flags & 2) bv[1] = gm_ld<DT>(a.bias2, n);
+  }
+  int ib = 0, is = 0;   // the next stage to load, and its buffer
+  auto issue = [&]() {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) tg_dma16(gb[i] + (long long)is * RB, voff[i], ldst[i] + (unsigned)(ib * SB));
+    ++is;
+    ib = ib + 1 == ST ? 0 : ib + 1;
+  };
+  tg_f32x4 acc[NW][TJ][TI];
+#pragma unroll
+  for (int u = 0; u < NW; ++u)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int i = 0; i < TI; ++i) acc[u][j][i] = tg_f32x4{0.f, 0.f, 0.f, 0.f};
+  // fragments: lane -> row lane % 16, chunk lane / 16 (+ 4 for the second half of a stage); a
+  // multiple of 16 rows leaves the slot permutation unchanged, so it is one offset per lane
+  const int fr = lane & 15, fc = lane >> 4;
+  const int fo[2] = {fr * RB + ((fc ^ ((fr >> 1) & 7)) * 16), fr * RB + (((fc + 4) ^ ((fr >> 1) & 7)) * 16)};
+#pragma unroll
+  for (int st = 0; st < ST - 1; ++st)
+    if (st < nsteps) issue();
+  int cb = 0;
+  for (int s = 0; s < nsteps; ++s) {
+    // stage s has landed when at most the stages issued after it are outstanding
+    gm_vmcnt_after<NI, ST - 2>(min(nsteps - 1 - s, ST - 2));
+    __syncthreads();                      // every wave's part of stage s is there, and every wave is done with s - 1
+    if (s + ST - 1 < nsteps) issue();     // into the buffer stage s - 1 used
+    const char* xs = Ls + cb * SB + wr * WM * RB;
+    const char* ws = Ls + cb * SB + (BM + wc * WN) * RB;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      uint4 fx[TI], fw[NW][TJ];
+#pragma unroll
+      for (int i = 0; i < TI; ++i) fx[i] = *(const uint4*)(xs + fo[k] + i * 16 * RB);
+#pragma unroll
+      for (int u = 0; u < NW; ++u)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) fw[u][j] = *(const uint4*)(ws + fo[k] + (u * BN + j * 16) * RB);
+      __builtin_amdgcn_s_setprio(1);   // a wave with its fragments goes ahead of one still reading (1-3%)
+#pragma unroll
+      for (int u = 0; u < NW; ++u)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+          for (int i = 0; i < TI; ++i) acc[u][j][i] = tg_mfma<DT>(fw[u][j], fx[i], acc[u][j][i]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    cb = cb + 1 == ST ? 0 : cb + 1;
+  }
+
+  // this lane's part of a 16 x 16 tile: row fr, columns cn .. cn + 3
+  const int cn = 4 * fc;
+  if (a.ksplit > 1) {
+#pragma unroll
+    for (int u = 0; u < NW; ++u)
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const int m = m_base + wr * WM + i * 16 + fr;
+        if (m >= M) continue;
+        float* p = a.part + (((long long)kz * NW + u) * a.M + m) * N;
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+          const int n = n_base + wc * WN + j * 16 + cn;
+          if ((N & 3) == 0) {
+            if (n < N) *(tg_f32x4*)(p + n) = acc[u][j][i];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) p[n + e] = acc[u][j][i][e];
+          }
+        }
+      }
+    return;
+  }
+  // epilogue: the rounded tile through LDS (round(acc + bias) is the first rounding point, so a
+  // 16-bit value holds it), then 16-byte row chunks; the residual's chunks are loaded first
+  uint16_t* T = (uint16_t*)Ls;
+  constexpr int CPR = BN / 8, CH = (BM * CPR + NTH - 1) / NTH;   // chunks per row, chunks per thread
+  const bool vec = (N & 7) == 0 && (a.ldo & 7) == 0 && ((size_t)a.out & 15) == 0 &&
+                   (EPI != GE_RESID || ((a.ldr & 7) == 0 && ((size_t)a.resid & 15) == 0));
+  uint4 rv[EPI == GE_RESID ? CH : 1];
+  if constexpr (EPI == GE_RESID) {
+    if (vec) {
+#pragma unroll
+      for (int k = 0; k < CH; ++k) {
+        const int idx = min(tid + NTH * k, BM * CPR - 1), r = idx / CPR, q = idx - r * CPR;
+        rv[k] = *(const uint4*)((const uint16_t*)a.resid + (long long)min(m_base + r, M - 1) * a.ldr +
+                                min(n_base + q * 8, N - 8));
+      }
+    }
+  }
+  if (tid < BN) {
+#pragma unroll
+    for (int u = 0; u < NW; ++u) Fb[u * BN + tid] = bv[u];
+  }
+  __syncthreads();   // every wave is done with the operand buffers
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    const int nl = wc * WN + j * 16 + cn;
+    const tg_f32x4 b0 = *(const tg_f32x4*)&Fb[nl];
+    tg_f32x4 b1{};
+    if constexpr (NW == 2) b1 = *(const tg_f32x4*)&Fb[BN + nl];
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const tg_f32x4 v = acc[0][j][i] + b0;
+      uint2 h = make_uint2(gm_pack2<DT>(v[0], v[1]), gm_pack2<DT>(v[2], v[3]));
+      if constexpr (EPI == GE_SILU) {
+        const tg_f32x4 w = acc[NW - 1][j][i] + b1;
+        const uint2 up = make_uint2(gm_pack2<DT>(w[0], w[1]), gm_pack2<DT>(w[2], w[3]));
+        const uint2 sg = make_uint2(gm_pack2<DT>(gm_silu(gm_lo<DT>(h.x)), gm_silu(gm_hi<DT>(h.x))),
+                                    gm_pack2<DT>(gm_silu(gm_lo<DT>(h.y)), gm_silu(gm_hi<DT>(h.y))));
+        h = make_uint2(gm_pack2<DT>(gm_lo<DT>(sg.x) * gm_lo<DT>(up.x), gm_hi<DT>(sg.x) * gm_hi<DT>(up.x)),
+                       gm_pack2<DT>(gm_lo<DT>(sg.y) * gm_lo<DT>(up.y), gm_hi<DT>(sg.y) * gm_hi<DT>(up.y)));
+      }
+      *(uint2*)&T[(wr * WM + i * 16 + fr) * TLD + nl] = h;
+    }
+  }
+  __syncthreads();
+  uint16_t* OUT = (uint16_t*)a.out;
+#pragma unroll
+  for (int k = 0; k < CH; ++k) {
+    const int idx = tid + NTH * k, r = idx / CPR, q = idx - r * CPR;
+    const int m = m_base + r, n0 = n_base + q * 8;
+    if (idx >= BM * CPR || m >= M || n0 >= N) continue;
+    const uint4 tv = *(const uint4*)&T[r * TLD + q * 8];
+    uint32_t tw[4] = {tv.x, tv.y, tv.z, tv.w};
+    if (vec) {
+      if constexpr (EPI == GE_RESID) {
+        const uint32_t rw[4] = {rv[k].x, rv[k].y, rv[k].z, rv[k].w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          tw[c] = gm_pack2<DT>(gm_lo<DT>(rw[c]) + gm_lo<DT>(tw[c]), gm_hi<DT>(rw[c]) + gm_hi<DT>(tw[c]));
+      }
+      *(uint4*)(OUT + (long long)m * a.ldo + n0) = make_uint4(tw[0], tw[1], tw[2], tw[3]);
+    } else {   // rows that are no multiple of 16 bytes, or unaligned: one value at a time
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (n0 + e >= N) continue;
+        float v = (e & 1) ? gm_hi<DT>(tw[e >> 1]) : gm_lo<DT>(tw[e >> 1]);
+        if constexpr (EPI == GE_RESID) v = gm_ld<DT>(a.resid, (long long)m * a.ldr + n0 + e) + v;
+        OUT[(long long)m * a.ldo + n0 + e] = gm_pack<DT>(v);
+      }
+    }
+  }
+}
+
+// k_gemm_<dtype>_<epilogue>_m<BM>n<BN>_w<waves>_k64d (BN columns per weight); the grouped kernels keep
+// the names of the tiles they are
+#define TILE_KERNEL(NAME, DT, EPI, NW, BM, BN, WR, WC, ST)                                        \
+  extern "C" __global__ void __launch_bounds__(64 * WR * WC) NAME(const GemmArgs a) {             \
+    tile_body<DT, EPI, NW, BM, BN, WR, WC, ST>(a);                                                \
+  }
+#define TILE_GRP(NAME, DT, BM, BN, WR, WC, ST)                                                    \
+  extern "C" __global__ void __launch_bounds__(64 * WR * WC) NAME(const GemmArgs a) {             \
+    tile_body<DT, GE_BIAS, 1, BM, BN, WR, WC, ST, true>(a);                                       \
+  }
+#define TILE_BIAS(DTN, DT)                                                                        \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m64n64_w8_k64d, DT, GE_BIAS, 1, 64, 64, 4, 2, 8)                \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m64n96_w8_k64d, DT, GE_BIAS, 1, 64, 96, 4, 2, 6)                \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m128n96_w8_k64d, DT, GE_BIAS, 1, 128, 96, 4, 2, 5)              \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m128n128_w8_k64d, DT, GE_BIAS, 1, 128, 128, 2, 4, 4)            \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m256n128_w8_k64d, DT, GE_BIAS, 1, 256, 128, 4, 2, 3)            \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m256n256_w8_k64d, DT, GE_BIAS, 1, 256, 256, 2, 4, 2)
+TILE_BIAS(bf16, HS_BF16)
+TILE_BIAS(f16, HS_F16)
+TILE_KERNEL(k_gemm_bf16_resid_m64n64_w8_k64d, HS_BF16, GE_RESID, 1, 64, 64, 4, 2, 8)
+TILE_KERNEL(k_gemm_bf16_resid_m64n96_w8_k64d, HS_BF16, GE_RESID, 1, 64, 96, 4, 2, 6)
+TILE_KERNEL(k_gemm_bf16_resid_m128n96_w8_k64d, HS_BF16, GE_RESID, 1, 128, 96, 4, 2, 5)
+TILE_KERNEL(k_gemm_bf16_resid_m128n128_w8_k64d, HS_BF16, GE_RESID, 1, 128, 128, 2, 4, 4)
+TILE_KERNEL(k_gemm_bf16_resid_m256n128_w8_k64d, HS_BF16, GE_RESID, 1, 256, 128, 4, 2, 3)
+TILE_KERNEL(k_gemm_bf16_resid_m256n256_w8_k64d, HS_BF16, GE_RESID, 1, 256, 256, 2, 4, 2)
+TILE_KERNEL(k_gemm_bf16_silu_m64n64_w8_k64d, HS_BF16, GE_SILU, 2, 64, 64, 2, 4, 6)
+TILE_KERNEL(k_gemm_bf16_silu_m128n144_w12_k64d, HS_BF16, GE_SILU, 2, 128, 144, 4, 3, 3)
+TILE_KERNEL(k_gemm_bf16_silu_m256n144_w12_k64d, HS_BF16, GE_SILU, 2, 256, 144, 4, 3, 2)
+TILE_GRP(k_gemm_bf16_grp_m64n64_k64d, HS_BF16, 64, 64, 4, 2, 8)
+TILE_GRP(k_gemm_bf16_grp_m64n128_k64d, HS_BF16, 64, 128, 2, 4, 6)
+TILE_GRP(k_gemm_bf16_grp_m128n128_k64d, HS_BF16, 128, 128, 2, 4, 4)

@@ -879,7 +879,7 @@ def qkv_rope_prefill(low) -> None:
 
 
 def _emit_qkv_prefill(low, xname, q, k, v, names) -> None:
-    from hip_compiler.subgraph_analyzer import gemm_tiling
+    from hip_compiler.subgraph_analyzer import gemm_tiling, tile_group, tile_plan
     x = low.aligned16(low.contiguous(xname), xname)   # a pending RMSNorm is materialised here
     rope = q["rope"]
     inv = low.contiguous(rope.inputs[0].name)
@@ -893,12 +893,15 @@ def _emit_qkv_prefill(low, xname, q, k, v, names) -> None:
         raise NotImplementedError("prefill RoPE reads int64 or int32 positions")
     N = (H + 2 * KVH) * D
     n1, n2 = H * D, (H + KVH) * D
-    bm, bn, _, dma = gemm_tiling(T, N, K)
-    if n1 % bn or n2 % bn:
-        bn = 64
-    bk = 64 if K % 64 == 0 else 32
-    if bm == 64 and bn == 128:   # grouped kernels come in 64 x 64 and 128 x 128
-        bn = 64
+    dma = K % 64 == 0
+    if dma:
+        bm, bn, waves, _ = tile_plan(T, N, K, "grp", (n1, n2))
+        bk, gn = 64, tile_group(T, N, bm, bn, 1, 1)
+    else:   # grouped kernels with register staging come in 64 x 64 and 128 x 128
+        bm, bn, _ = gemm_tiling(T, N, K)
+        if n1 % bn or n2 % bn or (bm == 64 and bn == 128):
+            bn = 64
+        bk, waves, gn = 32, 4, 1
     ws = [low.aligned16(low.contiguous(e["w"].name), e["w"].name) for e in (q, k, v)]
     bs = [low.contiguous(e["b"].name) if e["b"] is not None else None for e in (q, k, v)]
     y = low.new_storage(q["out"] + ".qkv", [T, N], "bfloat16")
@@ -906,12 +909,11 @@ def _emit_qkv_prefill(low, xname, q, k, v, names) -> None:
                 bias=low.ref(bs[0]) if bs[0] else None, bias2=low.ref(bs[1]) if bs[1] else None,
                 bias3=low.ref(bs[2]) if bs[2] else None, resid=None, out=low.ref(y), part=None,
                 M=T, ldx=K, ldw=K, ldo=N, ldr=N, sx=0, sw=0, so=0, batch=1, bdiv=1, N=N, K=K,
-                flags=1 if bs[0] else 0, ksplit=1, kchunk=K, nw=1, n1=n1, n2=n2)
+                flags=1 if bs[0] else 0, ksplit=1, kchunk=K, nw=1, n1=n1, n2=n2, gn=gn)
     ins = [xname] + [e["w"].name for e in (q, k, v)] + [e["b"].name for e in (q, k, v) if e["b"] is not None]
-    low.emit(LaunchStep(kind="gemm", kernel=f"k_gemm_bf16_grp_m{bm}n{bn}" + ("_k64d" if dma else "_k64" if bk == 64
-                                                                               else ""),
-                        module="gemm", arg_struct="GemmArgs", args=args,
-                        grid=((N + bn - 1) // bn, (T + bm - 1) // bm, 1), inputs=ins, outputs=[y.storage],
+    low.emit(LaunchStep(kind="gemm", kernel=f"k_gemm_bf16_grp_m{bm}n{bn}" + ("_k64d" if dma else ""),
+                        module="tile" if dma else "gemm", arg_struct="GemmArgs", args=args,
+                        grid=((N + bn - 1) // bn, (T + bm - 1) // bm, 1), block=(64 * waves, 1, 1), inputs=ins, outputs=[y.storage],
                         params={"M": T, "N": N, "K": K, "epilogue": "bias", "groups": [n1, n2], "mfma": True,
                                 "tile": (bm, bn), "ksplit": 1, "bk": bk, "lds_direct": dma, "nodes": names}))
     qo = low.new_storage(q["out"], [1, H, T, D], "bfloat16")

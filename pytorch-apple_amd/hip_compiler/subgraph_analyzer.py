@@ -61,60 +61,89 @@ WIDE_TA = 5
 WIDE_HALVES = os.environ.get("HIPRT_WIDE_HALVES", "1") == "1"
 GEMM_TARGET_WGS = 256    # workgroups a GEMM launch should reach (one per CU)
 GEMM_MIN_KCHUNK = 256    # smallest K range of one split-K workgroup
-GEMM_DMA_MAX_TILES = 1024   # tile grids at least this large keep register staging (gemm_tiling)
 CONV_D2_MAX_K = int(os.environ.get("HIPRT_CONV_D2_MAX_K", "1024"))   # convs up to this K: 2-stage staging
 CONV_D1_MAX_K = int(os.environ.get("HIPRT_CONV_D1_MAX_K", "64"))   # emit_conv_nhwc: one-stage 64x64 kernels up to this K
 CONV_SMALL_TILE_MAX_K = 512   # conv_gemm_tiling: 64 x 64 tiles for K up to this over many tiles
 CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order by operand sizes (emit_conv_nhwc)
 
 
-def gemm_tiling(M: int, N: int, K: int, nw: int = 1) -> tuple[int, int, int, bool]:
-    """(BM, BN, split-K, direct-to-LDS) for an M x N x K MFMA GEMM (nw = 2: two weights, BN
-    columns of each).
+# tile.hip kernels: (BM, BN, waves) -> (us per K step of 64, us per round of workgroups), by the kind
+# of launch. Fitted on MI355X to the kernels alone over M = 40 .. 4096 against weights of 1536 x 8960,
+# 1536 x 1536, 2048 x 1536, 4096 x 1536, 8960 x 1536 (SiLU pairs) and 151936 x 1536: a launch takes
+# ceil(workgroups / 256) rounds of (K / 64 steps + fixed), 2 us, and with K split TILE_REDUCE: the
+# reduce's 4 us and 0.4 us per MB of fp32 partials; within 10% of what was measured at all of them.
+TILE_COST = {
+    "silu": {(64, 64, 8): (0.42, 1.4), (128, 144, 12): (1.0, 5.0), (256, 144, 12): (1.65, 8.0)},
+    "one": {(64, 64, 8): (0.24, 2.1), (64, 96, 8): (0.31, 2.1), (128, 96, 8): (0.45, 1.5), (128, 128, 8): (0.495, 2.8),
+            (256, 128, 8): (0.775, 4.9), (256, 256, 8): (1.55, 8.0)},
+    "grp": {(64, 64, 8): (0.24, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.495, 2.8)},
+}
+TILE_REDUCE = (4.0, 0.4e-6)   # us, us per byte of partials
+TILE_CUS = 256
+TILE_MAX_SPLIT = 16
+TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
 
-    Rules fitted to sweeps on MI355X at M = 512 (bf16, K step 64, split-K reduce pass
-    included). Direct-to-LDS staging (the ``_k64d`` kernels: operands land in LDS several
-    K steps ahead without passing through registers) needs K % 64 == 0; it pays wherever the
-    tile grid is not large enough to hide the operand latency by itself, i.e. below
-    GEMM_DMA_MAX_TILES tiles. Two weights (gate/up with the SiLU-mul epilogue): 64 x 64
-    tiles, 52 us against 57 for 128 x 64 without. One weight: the largest tile that still
-    gives >= 256 workgroups; long rows (K >= 4096) take 128 x 128 with up to 4 K splits
-    (down_proj 512 x 1536 x 8960: 26 us with 4 splits, 32 with 8), or, with fewer than 48 such
-    tiles, 64 x 64 with up to 8 (down_proj at M = 128, a 128-token prefill: 17.0 us on 64 x 64
-    with 8 splits, 18.2 on 64 x 128 with 8, 19.6 on 128 x 128 with 16, 29.0 with 4); other grids under 256
-    tiles split K toward ~384 workgroups (o_proj 512 x 1536 x 1536 on 64 x 64: 9.5 us with
-    2 splits, 12.9 unsplit). The lm_head (4,748 tiles of 128 x 128) keeps register staging:
-    324 us against 367."""
-    dma = K % 64 == 0
+
+def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follows: bool = False) -> tuple[int, int, int, int]:
+    """(BM, BN, waves, K splits) of the tile.hip kernel that TILE_COST expects to be fastest for an
+    M x N x K GEMM, K % 64 == 0. ``kind``: "silu" (two weights), "one", or "grp" (columns of several
+    weights: BN divides every group boundary in ``bounds``); only "one" splits K.
+    ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
+    (k_gemm_reduce_*_resid_norm), so it costs its bytes only. The line between
+    two tiles lies where the rounds of workgroups make the smaller one cheaper: SiLU at N = 8960,
+    K = 1536 takes 128 x 144 tiles up to M = 512 (252 workgroups, 32 us; 256 x 144 43) and
+    256 x 144 at 1000 (252 workgroups, 50 us; 128 x 144 60)."""
+    best = None
+    for (bm, bn, waves), (step, fixed) in TILE_COST[kind].items():
+        if any(b % bn for b in bounds):
+            continue
+        tiles = -(-M // bm) * -(-N // bn)
+        for ks in range(1, TILE_MAX_SPLIT + 1 if kind == "one" else 2):
+            steps = -(-(K // 64) // ks)
+            if ks > 1 and (steps * 64 < GEMM_MIN_KCHUNK or -(-(K // 64) // steps) != ks
+                           or ks * M * N * 4 > TILE_MAX_PART or tiles * ks > 2 * TILE_CUS):
+                continue
+            us = -(-tiles * ks // TILE_CUS) * (steps * step + fixed)
+            if ks > 1:
+                us += (0.0 if norm_follows else TILE_REDUCE[0]) + TILE_REDUCE[1] * ks * M * N * 4
+            if best is None or us < best[0]:
+                best = (us, (bm, bn, waves, ks))
+    return best[1]
+
+
+def tile_group(M: int, N: int, bm: int, bn: int, nw: int, ksplit: int) -> int:
+    """Column tiles per group of tile.hip's tile order: the contiguous share of the tiles that one of
+    the 8 XCDs runs is about square in operand bytes (down_proj 2000 x 1536 x 8960: 7 columns x 5 row
+    tiles instead of 2 x 16, 25 MB of operands per XCD instead of 39); where whole columns of tiles fit
+    the share, one column after the other."""
+    gx, gy = -(-N // bn), -(-M // bm)
+    share = -(-gx * gy * ksplit // 8)
+    g = max(1, min(gx, round((share * bm / (bn * nw)) ** 0.5)))
+    return 1 if g * gy <= share else g
+
+
+def gemm_tiling(M: int, N: int, K: int, nw: int = 1) -> tuple[int, int, int]:
+    """(BM, BN, split-K) for an M x N x K GEMM with K % 64 != 0 (gemm.hip, operands staged through
+    registers; nw = 2: two weights, BN columns of each): the largest tile that still gives >= 256
+    workgroups; other grids split K toward ~384 workgroups (fp32 partials, then a reduce applies the
+    epilogue), long rows (K >= 4096) at most 4 or 8 ways."""
     ntiles = lambda bm, bn: ((M + bm - 1) // bm) * ((N + bn - 1) // bn)
     if nw == 2:
-        if dma:
-            # 128 x 96 tiles (4 x 1 waves) where they still give a full round of workgroups: more
-            # MFMA work per operand byte than 64 x 64 (77 against 44 FLOP per staged byte), and a
-            # grid that fits one round at two per CU (M = 512, N = 8960: 376)
-            return (128, 96, 1, True) if ntiles(128, 96) >= GEMM_TARGET_WGS else (64, 64, 1, True)
         for bm, bn in ((128, 64), (64, 64)):
             if ntiles(bm, bn) >= GEMM_TARGET_WGS:
-                return bm, bn, 1, False
-        return 64, 64, 1, False
+                return bm, bn, 1
+        return 64, 64, 1
     for bm, bn in ((128, 128), (64, 128), (64, 64)):
-        t = ntiles(bm, bn)
-        if t >= GEMM_TARGET_WGS:
-            return bm, bn, 1, dma and t < GEMM_DMA_MAX_TILES
+        if ntiles(bm, bn) >= GEMM_TARGET_WGS:
+            return bm, bn, 1
+    t = ntiles(64, 64)
     if K >= 4096:
-        t = ntiles(128, 96)
-        if dma and t >= 48:
-            # 128 x 96 over 4 x 1 waves, up to 8 K splits toward one round of 512 workgroups (two per
-            # CU): down_proj 512 x 1536 x 8960 23.1 us + 5.3 reduce, against 28.6 + 4.6 on 128 x 128
-            # with 4 splits (one workgroup per CU)
-            return 128, 96, max(1, min(8, 512 // t, K // GEMM_MIN_KCHUNK)), dma
         t = ntiles(128, 128)
         if t >= 48:
-            return 128, 128, max(1, min(4, 384 // t, K // GEMM_MIN_KCHUNK)), dma
+            return 128, 128, max(1, min(4, 384 // t, K // GEMM_MIN_KCHUNK))
         t = ntiles(64, 64)
-        return 64, 64, max(1, min(8, (384 + t - 1) // t, K // GEMM_MIN_KCHUNK)), dma
-    t = ntiles(64, 64)
-    return 64, 64, max(1, min((384 + t - 1) // t, K // GEMM_MIN_KCHUNK)), dma
+        return 64, 64, max(1, min(8, (384 + t - 1) // t, K // GEMM_MIN_KCHUNK))
+    return 64, 64, max(1, min((384 + t - 1) // t, K // GEMM_MIN_KCHUNK))
 
 
 def _is_nhwc(v: TView) -> bool:
@@ -731,8 +760,15 @@ class Lowering:
             self.views[out_name] = o
             return
         nw = 2 if epi == "silu" else 1
-        bm, bn, ksplit, dma = gemm_tiling(M, N, K, nw)
-        bk = 64 if K % 64 == 0 else 32
+        dma = K % 64 == 0   # whole 128-byte stages: the direct-to-LDS kernels of tile.hip
+        bk, waves, gn = (64, 8, 1) if dma else (32, 4, 1)
+        if dma:
+            norm_follows = epi == "resid" and N <= 2048 and N % 8 == 0 and \
+                any(i["x"] == out_name for i in self.rms_info.values())
+            bm, bn, waves, ksplit = tile_plan(M, N, K, "silu" if nw == 2 else "one", norm_follows=norm_follows)
+            gn = tile_group(M, N, bm, bn, nw, ksplit)
+        else:
+            bm, bn, ksplit = gemm_tiling(M, N, K, nw)
         kchunk = K
         if ksplit > 1:
             kchunk = ((K // bk + ksplit - 1) // ksplit) * bk
@@ -743,16 +779,15 @@ class Lowering:
                     bias=self.ref(bias) if bias else None, bias2=self.ref(bv2) if bv2 else None,
                     resid=self.ref(r) if r else None, out=self.ref(o), part=part, M=M, ldx=K, ldw=K, ldo=N, ldr=N,
                     sx=0, sw=0, so=0, batch=1, bdiv=1,
-                    N=N, K=K, flags=(1 if bias else 0) | (2 if bv2 else 0), ksplit=ksplit, kchunk=kchunk, nw=nw)
+                    N=N, K=K, flags=(1 if bias else 0) | (2 if bv2 else 0), ksplit=ksplit, kchunk=kchunk, nw=nw, gn=gn)
         ins = [x_name, w_name] + [t for t in (b_name, resid, w2, b2) if t]
         params = {"M": M, "N": N, "K": K, "epilogue": epi, "has_bias": bias is not None, "weights": nw,
                   "transpose_b": True, "nodes": nodes, "mfma": True, "tile": (bm, bn), "ksplit": ksplit, "bk": bk,
                   "lds_direct": dma}
         self.emit(LaunchStep(
-            kind="gemm", kernel=f"k_gemm_{dt}_{epi}_m{bm}n{bn}" + ("_k64d" if dma else "_k64" if bk == 64 else ""),
-            module="gemm",
-            arg_struct="GemmArgs", args=args,
-            grid=((N + bn - 1) // bn, (M + bm - 1) // bm, ksplit), inputs=ins,
+            kind="gemm", kernel=f"k_gemm_{dt}_{epi}_m{bm}n{bn}" + (f"_w{waves}_k64d" if dma else ""),
+            module="tile" if dma else "gemm", arg_struct="GemmArgs", args=args,
+            grid=((N + bn - 1) // bn, (M + bm - 1) // bm, ksplit), block=(64 * waves, 1, 1), inputs=ins,
             outputs=[out_name + ".kpart" if ksplit > 1 else out_name], params=params))
         if ksplit > 1:
             self.emit(LaunchStep(

@@ -70,7 +70,8 @@ _struct("GemmArgs", [("x", P), ("w", P), ("w2", P), ("bias", P), ("bias2", P), (
                      ("ldr", LL), ("sx", LL), ("sw", LL), ("so", LL), ("batch", I), ("bdiv", I), ("N", I), ("K", I),
                      ("flags", I), ("ksplit", I), ("kchunk", I), ("nw", I), ("n1", I), ("n2", I), ("bn_w", P),
                      ("bn_b", P), ("bn_mean", P), ("bn_var", P), ("zero", P), ("eps", F), ("cH", I), ("cW", I),
-                     ("cCin", I), ("cHo", I), ("cWo", I), ("cKW", I), ("csh", I), ("csw", I), ("cph", I), ("cpw", I)])
+                     ("cCin", I), ("cHo", I), ("cWo", I), ("cKW", I), ("csh", I), ("csw", I), ("cph", I), ("cpw", I),
+                     ("gn", I), ("gpad", I)])
 _struct("ConvArgs", [("x", P), ("w", P), ("bias", P), ("bn_w", P), ("bn_b", P), ("bn_mean", P), ("bn_var", P),
                      ("resid", P), ("out", P), ("part", P), ("M", LL), ("N", I), ("Cin", I), ("H", I), ("W", I),
                      ("Cout", I), ("Ho", I), ("Wo", I), ("KH", I), ("KW", I), ("sh", I), ("sw", I), ("ph", I),

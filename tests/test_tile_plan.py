@@ -1,0 +1,37 @@
+"""The plan of the wide-workgroup GEMMs (hip_compiler tile_plan / tile_group) and their tile order, on the CPU."""
+
+import pytest
+
+
+def test_tile_order_covers_every_tile_once():
+    """The grouped tile order (tile.hip) over grids that do and do not divide by 8 or by the group:
+    every (row tile, column tile, split) exactly once."""
+    for gx, gy, gz, gn in ((11, 16, 1, 5), (63, 8, 1, 1), (16, 16, 1, 7), (1, 1, 1, 1), (13, 3, 5, 4), (7, 9, 2, 7)):
+        total, seen = gx * gy * gz, set()
+        per, tall = -(-total // 8), 8 if total % 8 == 0 else total % 8
+        for lin in range(total):
+            xcd, loc = lin % 8, lin // 8
+            t = xcd * per + loc if xcd < tall else tall * per + (xcd - tall) * (per - 1) + loc
+            kz, t2 = divmod(t, gx * gy)
+            g0 = t2 // (gn * gy) * gn
+            gw = min(gn, gx - g0)
+            t3 = t2 - g0 * gy
+            seen.add((t3 // gw, g0 + t3 % gw, kz))
+        assert seen == {(m, n, z) for m in range(gy) for n in range(gx) for z in range(gz)}
+
+
+@pytest.mark.parametrize("kind,bounds", [("one", ()), ("silu", ()), ("grp", (1536, 1792)), ("grp", (512, 576))])
+def test_plan_covers_the_product(kind, bounds):
+    """Any size: the tile is one of the kernels, splits tile K exactly and stay within the scratch limit,
+    groups lie within the grid."""
+    from hip_compiler.subgraph_analyzer import GEMM_MIN_KCHUNK, TILE_COST, TILE_MAX_PART, tile_group, tile_plan
+
+    for M in (1, 16, 33, 63, 64, 65, 129, 300, 1000, 4096, 70000):
+        for N in (1, 8, 96, 513, 1536, 2048, 8960, 151936):
+            for K in (64, 128, 320, 1536, 8960):
+                bm, bn, waves, ks = tile_plan(M, N, K, kind, bounds)
+                assert (bm, bn, waves) in TILE_COST[kind] and not any(b % bn for b in bounds)
+                chunk = -(-(K // 64) // ks) * 64
+                assert ks == 1 or (kind == "one" and (ks - 1) * chunk < K <= ks * chunk and chunk >= GEMM_MIN_KCHUNK
+                                   and ks * M * N * 4 <= TILE_MAX_PART)
+                assert 1 <= tile_group(M, N, bm, bn, 2 if kind == "silu" else 1, ks) <= -(-N // bn)
