@@ -71,14 +71,14 @@ CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order 
 # of launch. Fitted on MI355X to the kernels alone over M = 40 .. 4096 against weights of 1536 x 8960,
 # 1536 x 1536, 2048 x 1536, 4096 x 1536, 8960 x 1536 (SiLU pairs) and 151936 x 1536: a launch takes
 # ceil(workgroups / 256) rounds of (K / 64 steps + fixed), 2 us, and with K split TILE_REDUCE: the
-# reduce's 4 us and 0.4 us per MB of fp32 partials; within 10% of what was measured at all of them.
+# reduce's 4 us and 0.2 us per MB of fp32 partials; within 10% of what was measured at all of them.
 TILE_COST = {
     "silu": {(64, 64, 8): (0.42, 1.4), (128, 144, 12): (1.0, 5.0), (256, 144, 12): (1.65, 8.0)},
     "one": {(64, 64, 8): (0.24, 2.1), (64, 96, 8): (0.31, 2.1), (128, 96, 8): (0.45, 1.5), (128, 128, 8): (0.495, 2.8),
             (256, 128, 8): (0.775, 4.9), (256, 256, 8): (1.55, 8.0)},
     "grp": {(64, 64, 8): (0.24, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.495, 2.8)},
 }
-TILE_REDUCE = (4.0, 0.4e-6)   # us, us per byte of partials
+TILE_REDUCE = (4.0, 0.2e-6, 1.5)   # us, us per byte of partials, us for a second round of 8 splits' loads
 TILE_CUS = 256
 TILE_MAX_SPLIT = 16
 TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
@@ -106,6 +106,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
             us = -(-tiles * ks // TILE_CUS) * (steps * step + fixed)
             if ks > 1:
                 us += (0.0 if norm_follows else TILE_REDUCE[0]) + TILE_REDUCE[1] * ks * M * N * 4
+                us += TILE_REDUCE[2] if ks > 8 else 0.0
             if best is None or us < best[0]:
                 best = (us, (bm, bn, waves, ks))
     return best[1]
@@ -792,7 +793,7 @@ class Lowering:
         if ksplit > 1:
             self.emit(LaunchStep(
                 kind="gemm", kernel=f"k_gemm_reduce_{dt}_{epi}", module="gemm", arg_struct="GemmArgs",
-                args=dict(args), grid=grid1d(M * N), inputs=[out_name + ".kpart"] + ins[2:], outputs=[out_name],
+                args=dict(args), grid=grid1d(-(-M * N // 4)), inputs=[out_name + ".kpart"] + ins[2:], outputs=[out_name],
                 params=dict(params, reduce=True)))
         self.views[out_name] = o
 
@@ -1221,7 +1222,7 @@ class Lowering:
         if ksplit > 1:
             self.emit(LaunchStep(
                 kind="conv", kernel=f"k_gemm_reduce_{dts}_conv", module="gemm", arg_struct="GemmArgs",
-                args=dict(args), grid=grid1d(M * Cout), inputs=[out_name + ".kpart"] + ins[2:],
+                args=dict(args), grid=grid1d(-(-M * Cout // 4)), inputs=[out_name + ".kpart"] + ins[2:],
                 outputs=[out_name], params=dict(params, reduce=True)))
         self.views[out_name] = o
 
