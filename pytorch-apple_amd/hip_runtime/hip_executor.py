@@ -5,9 +5,10 @@ Init-time work: load code objects (AOT ``.hsaco`` and hiprtc-compiled chains),
 allocate the arena (zero-filled once), pack every step's argument struct with
 concrete arena pointers, and record where external buffers (graph inputs and
 weights) must be patched in. ``run()`` resolves the external pointers; when they
-match a set seen before, the HIP graph captured for that set is relaunched as-is
-(one host call per step, instead of the reference's one Python dispatch per IR
-step); a new set re-packs the affected kernargs and captures one more graph. Up to
+match the set packed last, the list is launched as it is (one host call per step,
+instead of the reference's one Python dispatch per IR step), launch by launch or, for
+long lists, as the HIP graph captured for that set; a new set re-packs the affected
+kernargs and, with graphs, captures one more. Up to
 ``MAX_GRAPHS`` graphs are kept, least recently used first out, so a loop whose
 first step reads one buffer and whose later steps read another (a decode loop
 feeding its own argmax back as ``input_ids``) captures twice in total, not twice
@@ -34,6 +35,13 @@ from hip_runtime.kernels import STRUCTS, ModuleCache
 
 _MODULES: dict[int, ModuleCache] = {}
 MAX_GRAPHS = 8
+# launch lists shorter than this are launched one by one (hs_replay), longer ones as one captured
+# graph. One call after the other, direct against graph: 2 launches (the MLP block of one token) 16.9
+# against 22.1 us, 3-4 (128 / 1000 rows) 44.9 / 96 against 46.0 / 104, 22 (two prefill layers of 2000
+# tokens) 732 against 769; 38 and 62 (prefill with the full head) 465 / 1056 against 471 / 1061, 80
+# (ResNet-50 at batch 1) 493 against 487. A call that is waited for: 2 launches 30 against 44 us,
+# 62 and 80 1086 / 526 against 1076 / 516, where the host's 1.5 us per launch begins to show.
+GRAPH_MIN_STEPS = 33
 MAX_TABLES = 8   # pointer tables kept per executor without graphs (with graphs: all)
 
 
@@ -94,9 +102,9 @@ class HIPExecutor:
         self.program = program
         self.device = backend.device if backend is not None else torch.device("cuda", torch.cuda.current_device())
         if use_graph is None:
-            # a graph pays for a launch list; around one launch (the persistent decode step) it only
-            # adds to the gap between launches (0.680 -> 0.677 ms per decode step launched directly)
-            use_graph = os.environ.get("HIPRT_NO_GRAPH", "0") != "1" and len(program.steps) > 1
+            # a graph saves host time per launch and costs about 15 us before its first kernel: it pays
+            # for long lists only (GRAPH_MIN_STEPS)
+            use_graph = os.environ.get("HIPRT_NO_GRAPH", "0") != "1" and len(program.steps) >= GRAPH_MIN_STEPS
         self.use_graph = use_graph
         mods = module_cache(self.device.index or 0)
         gen = {ks.kernel_name: ks.source_code for ks in program.kernel_sources}
@@ -149,6 +157,7 @@ class HIPExecutor:
         # new set patches its kernargs without building a name -> pointer map
         pos = {n: (0, i) for i, n in enumerate(self._w_names)} | {n: (1, i) for i, n in enumerate(self._in_names)}
         self._fix_pos = [(s, field, idx, *pos[storage], off) for s, field, idx, storage, off in self._fixups]
+        self._fix_in = [f for f in self._fix_pos if f[3] == 1]   # those a change of inputs alone touches
         self._w_src, self._w_snap, self._w_key = None, (), ()
         self._last_bufs: tuple | None = None      # input buffer objects of the previous launch
         self._last_in_key: tuple = ()
@@ -200,7 +209,10 @@ class HIPExecutor:
             arr[idx] = val
 
     def _patch(self, key: tuple) -> None:
-        for s, field, idx, part, i, off in self._fix_pos:
+        # a list launched directly is re-packed whenever the pointer set changes: with the weights packed
+        # now, only the inputs' pointers
+        same_w = self._ext_key is not None and self._ext_key[0] == key[0]
+        for s, field, idx, part, i, off in self._fix_in if same_w else self._fix_pos:
             val = key[part][i] + off
             if idx < 0:
                 setattr(s, field, val)
