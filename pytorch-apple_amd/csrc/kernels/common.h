@@ -539,7 +539,8 @@ struct PrefillAttnArgs {      // causal / masked attention of T queries over S k
   int mask_dtype;             // -1: no mask
   int add_dtype;              // rounding dtype of (scores + mask)
   int dtype;                  // bf16 or fp16
-  const int* blk_limit;       // per 32-query block: position blocks to visit (k_mask_extent), or null: all
+  const int* blk_limit;       // per 32-query block (k_mask_extent): position blocks to visit, and how many of
+                              //   the first are open for every row; or null: all of them, none known open
 };
 
 struct ReduceNormArgs {       // split-K reduce + residual, then RMSNorm of the result (gemm.hip)
@@ -562,7 +563,7 @@ struct ReduceNormArgs {       // split-K reduce + residual, then RMSNorm of the 
 
 struct MaskExtentArgs {       // k_mask_extent: last open mask column of each block of 32 query rows
   const void* mask;           // element (t, s) at t*row_stride + s*col_stride
-  int* nblk_out;              // [ceil(T / 32)]: 1 + (last column != -inf) / 32, 0 when none
+  int* nblk_out;              // [ceil(T / 32)][2]: 1 + (last column != -inf) / 32, 0 when none; (first column != 0) / 32
   long long T;
   long long S;
   long long row_stride;
@@ -944,7 +945,7 @@ __device__ __forceinline__ float block_max256(float v, float* red) {
 #endif
 
 #if defined(__HIPCC__) && !defined(__HIPCC_RTC__)
-// ---------------------------------------------------------------- MFMA GEMM helpers (gemm.hip, tile.hip)
+// ---------------------------------------------------------------- MFMA helpers (gemm.hip, tile.hip, attention.hip)
 
 enum { GE_BIAS = 0, GE_RESID = 1, GE_SILU = 2, GE_CONV = 3 };
 
@@ -994,6 +995,12 @@ __device__ __forceinline__ float gm_silu(float v) {
   const float d = 0.25f + __builtin_amdgcn_exp2f(__builtin_fmaf(v, -1.44269504088896340736f, -2.f));
   const float v4 = 0.25f * v, r = __builtin_amdgcn_rcpf(d), q = v4 * r, rem = __builtin_fmaf(-q, d, v4);
   return (rem < 0.f || rem > 0.f) ? __builtin_fmaf(rem, r, q) : q;
+}
+
+// 16 bytes per lane from base + off into LDS at lds + 16 * lane. Inline assembly, so that the compiler
+// does not wait for it before every LDS read; the waits are explicit (gm_vmcnt, gm_vmcnt_after).
+__device__ __forceinline__ void gm_dma16s(const void* base, unsigned off, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
 
 // s_waitcnt vmcnt(N), the other counters untouched

@@ -49,12 +49,6 @@ __device__ __forceinline__ tg_f32x4 tg_mfma(const uint4 a, const uint4 b, tg_f32
                                                   c, 0, 0, 0);
 }
 
-// 16 bytes per lane from base + off into LDS at lds + 16 * lane. Inline assembly, so that the compiler
-// does not wait for it before every LDS read; the waits are explicit (gm_vmcnt_after).
-__device__ __forceinline__ void tg_dma16(const void* base, unsigned off, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-
 template <int DT, int EPI, int NW, int BM, int BN, int WR, int WC, int ST, bool GRP = false>
 __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   constexpr int NWV = WR * WC, NTH = 64 * NWV, BNT = BN * NW;
@@ -125,7 +119,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   int ib = 0, is = 0;   // the next stage to load, and its buffer
   auto issue = [&]() {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) tg_dma16(gb[i] + (long long)is * RB, voff[i], ldst[i] + (unsigned)(ib * SB));
+    for (int i = 0; i < NI; ++i) gm_dma16s(gb[i] + (long long)is * RB, voff[i], ldst[i] + (unsigned)(ib * SB));
     ++is;
     ib = ib + 1 == ST ? 0 : ib + 1;
   };

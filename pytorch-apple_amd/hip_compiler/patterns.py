@@ -28,6 +28,11 @@ from npu_compiler.ir_reader import OpNode
 # kernel (k_gemm_reduce_*_resid_norm); off = two launches with the same results
 FUSE_REDUCE_NORM = True
 
+# workgroups of prefill attention up to which a workgroup takes fewer heads (one per CU; 512 tokens of
+# 12 heads 13.5 us with one head
+# each, 18.6 with three; 2000 tokens 51 with three, in 252 workgroups)
+PREFILL_ATTN_WGS = 256
+
 _PASS = ("aten._assert_tensor_metadata.default",)
 
 
@@ -347,22 +352,26 @@ def _emit_prefill_attention(low, q, k, v, mask, out, scale, H, kvh, S, T, add_dt
                 dtype=DTYPE_CODE[dt], **margs)
     kname = "k_attn_prefill" + ("" if dt == "bfloat16" else "_f16") + \
         ("_nomask" if mask is None else ("_f32mask" if margs["mask_dtype"] == DTYPE_CODE["float32"] else ""))
-    low.emit(LaunchStep(kind="attention", kernel=kname,
-                        module="attention", arg_struct="PrefillAttnArgs", args=args, grid=((T + 31) // 32, H, 1),
-                        inputs=[q, k, v] + ([mask] if mask else []), outputs=[out.name],
+    # query heads of one KV head per workgroup (they share its K and V blocks in LDS): the fewest
+    # that still give one workgroup per CU, else the most
+    hws = [n for n in (1, 2, 3) if (H // kvh) % n == 0]
+    hw = next((n for n in hws if (T + 31) // 32 * (H // n) <= PREFILL_ATTN_WGS), hws[-1])
+    low.emit(LaunchStep(kind="attention", kernel=kname + ("" if hw == 1 else f"_h{hw}"),
+                        module="attention", arg_struct="PrefillAttnArgs", args=args, grid=((T + 31) // 32, H // hw, 1),
+                        block=(256 * hw, 1, 1), inputs=[q, k, v] + ([mask] if mask else []), outputs=[out.name],
                         params={"T": T, "S": S, "heads": H, "kv_heads": kvh, "nodes": names}))
     low.views[out.name] = st.with_(shape=(1, H, T, D), strides=(T * H * D, D, H * D, 1))
 
 
 def _mask_extent(low, name: str, mv, row: int, T: int, S: int):
-    """Per block of 32 query rows, how many 32-position blocks the mask leaves open at most
-    (``k_mask_extent``), computed once per distinct mask view and shared by every layer's
-    prefill attention."""
+    """Per block of 32 query rows, how many 32-position blocks the mask leaves open at most and how
+    many of the first it leaves untouched (``k_mask_extent``), computed once per distinct mask view
+    and shared by every layer's prefill attention."""
     key = (mv.storage, mv.offset, tuple(mv.shape), tuple(mv.strides), row, T, S)
     ref = low.mask_extents.get(key)
     if ref is None:
         nqb = (T + 31) // 32
-        ref = low.scratch(name + ".extent", 4 * nqb)
+        ref = low.scratch(name + ".extent", 8 * nqb)
         low.emit(LaunchStep(kind="special", kernel="k_mask_extent", module="attention", arg_struct="MaskExtentArgs",
                             args=dict(mask=low.ref(mv), nblk_out=ref, T=T, S=S, row_stride=row,
                                       col_stride=mv.strides[-1], mask_dtype=DTYPE_CODE[mv.dtype]),

@@ -78,7 +78,9 @@ TILE_COST = {
             (256, 128, 8): (0.775, 4.9), (256, 256, 8): (1.55, 8.0)},
     "grp": {(64, 64, 8): (0.24, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.495, 2.8)},
 }
-TILE_REDUCE = (4.0, 0.2e-6, 1.5)   # us, us per byte of partials, us for a second round of 8 splits' loads
+# us, us per byte of partials, per split (o_proj 128 x 1536 x 1536: 9.3 us with 4 splits, 9.9 with 5),
+# and for a second round of 8 splits' loads
+TILE_REDUCE = (4.0, 0.2e-6, 0.15, 1.5)
 TILE_CUS = 256
 TILE_MAX_SPLIT = 16
 TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
@@ -89,7 +91,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
     M x N x K GEMM, K % 64 == 0. ``kind``: "silu" (two weights), "one", or "grp" (columns of several
     weights: BN divides every group boundary in ``bounds``); only "one" splits K.
     ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
-    (k_gemm_reduce_*_resid_norm), so it costs its bytes only. The line between
+    (k_gemm_reduce_*_resid_norm), so it costs little more than its bytes. The line between
     two tiles lies where the rounds of workgroups make the smaller one cheaper: SiLU at N = 8960,
     K = 1536 takes 128 x 144 tiles up to M = 512 (252 workgroups, 32 us; 256 x 144 43) and
     256 x 144 at 1000 (252 workgroups, 50 us; 128 x 144 60)."""
@@ -105,8 +107,8 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
                 continue
             us = -(-tiles * ks // TILE_CUS) * (steps * step + fixed)
             if ks > 1:
-                us += (0.0 if norm_follows else TILE_REDUCE[0]) + TILE_REDUCE[1] * ks * M * N * 4
-                us += TILE_REDUCE[2] if ks > 8 else 0.0
+                us += (1.5 if norm_follows else TILE_REDUCE[0]) + TILE_REDUCE[1] * ks * M * N * 4
+                us += TILE_REDUCE[2] * ks + (TILE_REDUCE[3] if ks > 8 else 0.0)
             if best is None or us < best[0]:
                 best = (us, (bm, bn, waves, ks))
     return best[1]
