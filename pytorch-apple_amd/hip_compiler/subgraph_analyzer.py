@@ -1383,7 +1383,8 @@ class Lowering:
             self.emit(LaunchStep(
                 kind="reduction", kernel=f"k_mean_nhwc_{'bf16' if xv.dtype == 'bfloat16' else 'f16'}", module="conv",
                 arg_struct="MeanNHWCArgs", args=dict(x=self.ref(xv), out=self.ref(o), n=N, hw=H * W, c=C),
-                grid=grid1d(N * C // 8), inputs=[node.inputs[0].name], outputs=[out.name], params={"nhwc": True}))
+                grid=grid1d(N * -(-C // 64), 4), inputs=[node.inputs[0].name], outputs=[out.name],
+                params={"nhwc": True}))
             self.views[out.name] = o
             return
         x = self.contiguous(node.inputs[0].name)
