@@ -997,6 +997,24 @@ __device__ __forceinline__ float gm_silu(float v) {
   return (rem < 0.f || rem > 0.f) ? __builtin_fmaf(rem, r, q) : q;
 }
 
+// conv epilogue (conv.hip's rounding points): after v = round(acc + bias),
+//   batch norm: v = round(v * al + be), al = w / sqrt(var + eps), be = bias - mean * al;
+//   residual: v = round(v + r);  ReLU: v = max(v, 0) (NaN kept)
+template <int DT>
+__device__ __forceinline__ void gm_bn_factors(const GemmArgs& a, int n, float& al, float& be) {
+  const float g = gm_ld<DT>(a.bn_w, n), bb = gm_ld<DT>(a.bn_b, n);
+  const float mu = gm_ld<DT>(a.bn_mean, n), var = gm_ld<DT>(a.bn_var, n);
+  al = g / sqrtf(var + a.eps);
+  be = bb - mu * al;
+}
+template <int DT>
+__device__ __forceinline__ float gm_conv_tail_f(const GemmArgs& a, float v, float al, float be, float r) {
+  if (a.flags & 2) v = gm_round<DT>(v * al + be);
+  if (a.flags & 4) v = gm_round<DT>(v + r);
+  if (a.flags & 8) v = v != v ? v : fmaxf(v, 0.f);
+  return v;
+}
+
 // 16 bytes per lane from base + off into LDS at lds + 16 * lane. Inline assembly, so that the compiler
 // does not wait for it before every LDS read; the waits are explicit (gm_vmcnt, gm_vmcnt_after).
 __device__ __forceinline__ void gm_dma16s(const void* base, unsigned off, unsigned lds) {

@@ -54,23 +54,6 @@ __device__ __forceinline__ int gm_swz(int r) { return GM_SWZ_PAIR ? (r >> 1) & 7
 __device__ __forceinline__ void gm_dma16(const void* g, unsigned lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
 }
-// conv epilogue (conv.hip's rounding points): after v = round(acc + bias),
-//   batch norm: v = round(v * al + be), al = w / sqrt(var + eps), be = bias - mean * al;
-//   residual: v = round(v + r);  ReLU: v = max(v, 0) (NaN kept)
-template <int DT>
-__device__ __forceinline__ void gm_bn_factors(const GemmArgs& a, int n, float& al, float& be) {
-  const float g = gm_ld<DT>(a.bn_w, n), bb = gm_ld<DT>(a.bn_b, n);
-  const float mu = gm_ld<DT>(a.bn_mean, n), var = gm_ld<DT>(a.bn_var, n);
-  al = g / sqrtf(var + a.eps);
-  be = bb - mu * al;
-}
-template <int DT>
-__device__ __forceinline__ float gm_conv_tail_f(const GemmArgs& a, float v, float al, float be, float r) {
-  if (a.flags & 2) v = gm_round<DT>(v * al + be);
-  if (a.flags & 4) v = gm_round<DT>(v + r);
-  if (a.flags & 8) v = v != v ? v : fmaxf(v, 0.f);
-  return v;
-}
 template <int DT>
 __device__ __forceinline__ float gm_conv_tail(const GemmArgs& a, float v, float al, float be, uint16_t r) {
   return gm_conv_tail_f<DT>(a, v, al, be, DT == HS_BF16 ? bf16_to_f32(r) : f16_to_f32(r));
@@ -819,16 +802,7 @@ GEMM_KERNEL_K64(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64)
 #define GM_CONV_WPE 8
 #endif
 #define GM_ATTRS_CONV __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, GM_CONV_WPE)))
-#define GEMM_CONV(DTN, DT, BM, BN, ST)                                                                              \
-  extern "C" __global__ void GM_ATTRS k_gemm_##DTN##_conv_m##BM##n##BN##_k64(const GemmArgs a) {                    \
-    gemm_body<DT, GE_CONV, 1, BM, BN, false, 64>(a);                                                                \
-  }                                                                                                                 \
-  extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_conv_m##BM##n##BN##_k64d(const GemmArgs a) {              \
-    gemm_body<DT, GE_CONV, 1, BM, BN, false, 64, false, ST>(a);                                                     \
-  }                                                                                                                 \
-  extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_convg_m##BM##n##BN##_k64d(const GemmArgs a) {             \
-    gemm_body<DT, GE_CONV, 1, BM, BN, false, 64, false, ST, 1>(a);                                                  \
-  }                                                                                                                 \
+#define GEMM_CONV(DTN, DT, BM, BN)                                                                                  \
   extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_conv_m##BM##n##BN##_k64d2(const GemmArgs a) {             \
     gemm_body<DT, GE_CONV, 1, BM, BN, false, 64, false, 2>(a);                                                      \
   }                                                                                                                 \
@@ -838,6 +812,14 @@ GEMM_KERNEL_K64(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64)
   extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_convp_m##BM##n##BN##_k64d2(const GemmArgs a) {            \
     gemm_body<DT, GE_CONV, 1, BM, BN, false, 64, false, 2, 2>(a);                                                   \
   }
+// long K over few tiles (the wide tiles of long K run on tile.hip): four stages
+#define GEMM_CONV_D(DTN, DT)                                                                                        \
+  extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_conv_m64n64_k64d(const GemmArgs a) {                      \
+    gemm_body<DT, GE_CONV, 1, 64, 64, false, 64, false, 4>(a);                                                      \
+  }                                                                                                                 \
+  extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_convg_m64n64_k64d(const GemmArgs a) {                     \
+    gemm_body<DT, GE_CONV, 1, 64, 64, false, 64, false, 4, 1>(a);                                                   \
+  }
 // short K (1 x 1 convs over few channels): the LDS of one stage, 16 KB at 64 x 64, so up to eight
 // workgroups share a CU
 extern "C" __global__ void GM_ATTRS_CONV k_gemm_f16_conv_m64n64_k64d1(const GemmArgs a) {
@@ -846,14 +828,16 @@ extern "C" __global__ void GM_ATTRS_CONV k_gemm_f16_conv_m64n64_k64d1(const Gemm
 extern "C" __global__ void GM_ATTRS_CONV k_gemm_bf16_conv_m64n64_k64d1(const GemmArgs a) {
   gemm_body<HS_BF16, GE_CONV, 1, 64, 64, false, 64, false, 2, 0, 1>(a);
 }
-GEMM_CONV(f16, HS_F16, 128, 128, 4)
-GEMM_CONV(f16, HS_F16, 128, 64, 3)
-GEMM_CONV(f16, HS_F16, 64, 128, 3)
-GEMM_CONV(f16, HS_F16, 64, 64, 4)
-GEMM_CONV(bf16, HS_BF16, 128, 128, 4)
-GEMM_CONV(bf16, HS_BF16, 128, 64, 3)
-GEMM_CONV(bf16, HS_BF16, 64, 128, 3)
-GEMM_CONV(bf16, HS_BF16, 64, 64, 4)
+GEMM_CONV(f16, HS_F16, 128, 128)
+GEMM_CONV(f16, HS_F16, 128, 64)
+GEMM_CONV(f16, HS_F16, 64, 128)
+GEMM_CONV(f16, HS_F16, 64, 64)
+GEMM_CONV_D(f16, HS_F16)
+GEMM_CONV(bf16, HS_BF16, 128, 128)
+GEMM_CONV(bf16, HS_BF16, 128, 64)
+GEMM_CONV(bf16, HS_BF16, 64, 128)
+GEMM_CONV(bf16, HS_BF16, 64, 64)
+GEMM_CONV_D(bf16, HS_BF16)
 GEMM_REDUCE(k_gemm_reduce_f16_conv, HS_F16, GE_CONV)
 GEMM_REDUCE(k_gemm_reduce_bf16_conv, HS_BF16, GE_CONV)
 GEMM_KERNEL_GRP(k_gemm_bf16_grp_m64n64, HS_BF16, 64, 64)

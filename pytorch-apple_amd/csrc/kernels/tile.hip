@@ -31,6 +31,11 @@
 //   SILU  out = round(round(silu(round(acc_g + b_g))) * round(acc_u + b_u))   (NW = 2)
 // ksplit > 1: grid.z workgroups take kchunk of K each and store fp32 partials [z, NW, M, N]; a
 // k_gemm_reduce_* kernel (gemm.hip) sums them in order and applies the epilogue.
+//   CONV  round(acc + b), batch norm, residual and ReLU as gemm.hip's conv epilogue
+// CV: x rows are gathered from an NHWC image, one tap and 64 channels per stage (K = (kh, kw, ci),
+// cCin % 64 == 0), taps outside it from a.zero. ResNet-50's 3 x 3 convs at batch 32 with 128 / 256 / 512
+// channels: 23.0 / 26.8 / 26.4 -> 20.3 / 24.1 / 19.6 us against the 4-wave kernels; they take in 45-60 GB/s
+// per CU from the L2, which bounds them.
 // GRP: output columns [0, n1), [n1, n2), [n2, N) come from three weights and biases (n1, n2
 // multiples of BN), e.g. q | k | v of one activation.
 #include "common.h"
@@ -49,7 +54,12 @@ __device__ __forceinline__ tg_f32x4 tg_mfma(const uint4 a, const uint4 b, tg_f32
                                                   c, 0, 0, 0);
 }
 
-template <int DT, int EPI, int NW, int BM, int BN, int WR, int WC, int ST, bool GRP = false>
+// the same from a 64-bit address per lane
+__device__ __forceinline__ void tg_dma16v(const void* p, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory", "m0");
+}
+
+template <int DT, int EPI, int NW, int BM, int BN, int WR, int WC, int ST, bool GRP = false, bool CV = false>
 __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   constexpr int NWV = WR * WC, NTH = 64 * NWV, BNT = BN * NW;
   constexpr int WM = BM / WR, WN = BN / WC, TI = WM / 16, TJ = WN / 16;   // wave tile, in 16 x 16 MFMA tiles
@@ -60,7 +70,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   static_assert(ST * SB >= BM * TLD * 2 || ST == 2, "epilogue tile");
   constexpr int LDSB = ST * SB > BM * TLD * 2 ? ST * SB : BM * TLD * 2;
   __shared__ __attribute__((aligned(16))) char Ls[LDSB];
-  __shared__ __attribute__((aligned(16))) float Fb[NW * BN];
+  __shared__ __attribute__((aligned(16))) float Fb[(EPI == GE_CONV ? 3 : NW) * BN];   // bias per weight; conv: bias, al, be
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave / WC, wc = wave % WC;
   // XCD-aware tile order: workgroup L runs on XCD L % 8, so L is remapped to give each XCD a contiguous
@@ -91,13 +101,24 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   unsigned voff[NI];
   const char* gb[NI];
   unsigned ldst[NI];
+  // CV: the row's image, its pixel's first input row and column (padding: < 0), and the lane's chunk
+  int gim[CV ? NI : 1], ghi[CV ? NI : 1], gwi[CV ? NI : 1];
+  unsigned gch[CV ? NI : 1];
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)&Ls[0];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int q = min(wave + i * NWV, INS - 1), r = 8 * q + (lane >> 3);
     const unsigned chunk = (unsigned)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
     ldst[i] = lds0 + (unsigned)q * 1024u;
-    if (8 * q < BM) {
+    if (CV && 8 * q < BM) {   // lane pointer offsets are made per step (the taps)
+      const int HoWo = a.cHo * a.cWo, m = min(m_base + r, M - 1), n = m / HoWo, p = m - n * HoWo, ho = p / a.cWo;
+      ghi[i] = ho * a.csh - a.cph;
+      gwi[i] = (p - ho * a.cWo) * a.csw - a.cpw;
+      gim[i] = n;
+      gch[i] = chunk;
+      voff[i] = 0;
+      gb[i] = (const char*)a.x;
+    } else if (8 * q < BM) {
       gb[i] = (const char*)a.x + ((long long)m_base * a.ldx + kbeg) * 2;
       voff[i] = (unsigned)(min(m_base + r, M - 1) - m_base) * (unsigned)(a.ldx * 2) + chunk;
     } else {
@@ -117,9 +138,36 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
       if (a.flags & 2) bv[1] = gm_ld<DT>(a.bias2, n);
   }
   int ib = 0, is = 0;   // the next stage to load, and its buffer
+  int c0 = 0, kh = 0, kw = 0;   // CV: its channels and tap (64 channels of one tap per stage)
+  if constexpr (CV) {
+    const int tap = kbeg / a.cCin;
+    c0 = kbeg - tap * a.cCin;
+    kh = tap / a.cKW;
+    kw = tap - kh * a.cKW;
+  }
   auto issue = [&]() {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) gm_dma16s(gb[i] + (long long)is * RB, voff[i], ldst[i] + (unsigned)(ib * SB));
+    for (int i = 0; i < NI; ++i) {
+      const unsigned dst = ldst[i] + (unsigned)(ib * SB);
+      if (CV && 8 * min(wave + i * NWV, INS - 1) < BM) {   // uniform; taps outside the image read a.zero
+        const int hi = ghi[i] + kh, wi = gwi[i] + kw;
+        const bool ok = (unsigned)hi < (unsigned)a.cH && (unsigned)wi < (unsigned)a.cW;
+        const long long e = (((long long)gim[i] * a.cH + hi) * a.cW + wi) * a.cCin + c0;
+        tg_dma16v(ok ? (const char*)a.x + 2 * e + gch[i] : (const char*)a.zero, dst);
+      } else {
+        gm_dma16s(gb[i] + (long long)is * RB, voff[i], dst);
+      }
+    }
+    if constexpr (CV) {
+      c0 += 64;
+      if (c0 == a.cCin) {
+        c0 = 0;
+        if (++kw == a.cKW) {
+          kw = 0;
+          ++kh;
+        }
+      }
+    }
     ++is;
     ib = ib + 1 == ST ? 0 : ib + 1;
   };
@@ -195,10 +243,11 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   uint16_t* T = (uint16_t*)Ls;
   constexpr int CPR = BN / 8, CH = (BM * CPR + NTH - 1) / NTH;   // chunks per row, chunks per thread
   const bool vec = (N & 7) == 0 && (a.ldo & 7) == 0 && ((size_t)a.out & 15) == 0 &&
-                   (EPI != GE_RESID || ((a.ldr & 7) == 0 && ((size_t)a.resid & 15) == 0));
-  uint4 rv[EPI == GE_RESID ? CH : 1];
-  if constexpr (EPI == GE_RESID) {
-    if (vec) {
+                   (!(EPI == GE_RESID || (EPI == GE_CONV && (a.flags & 4))) || ((a.ldr & 7) == 0 && ((size_t)a.resid & 15) == 0));
+  constexpr bool HAS_R = EPI == GE_RESID || EPI == GE_CONV;
+  uint4 rv[HAS_R ? CH : 1];
+  if constexpr (HAS_R) {
+    if (vec && (EPI == GE_RESID || (a.flags & 4))) {
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         const int idx = min(tid + NTH * k, BM * CPR - 1), r = idx / CPR, q = idx - r * CPR;
@@ -210,6 +259,12 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   if (tid < BN) {
 #pragma unroll
     for (int u = 0; u < NW; ++u) Fb[u * BN + tid] = bv[u];
+    if constexpr (EPI == GE_CONV) {
+      float al = 1.f, be = 0.f;
+      if (a.flags & 2) gm_bn_factors<DT>(a, min(n_base + tid, N - 1), al, be);
+      Fb[BN + tid] = al;
+      Fb[2 * BN + tid] = be;
+    }
   }
   __syncthreads();   // every wave is done with the operand buffers
 #pragma unroll
@@ -249,6 +304,14 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
         for (int c = 0; c < 4; ++c)
           tw[c] = gm_pack2<DT>(gm_lo<DT>(rw[c]) + gm_lo<DT>(tw[c]), gm_hi<DT>(rw[c]) + gm_hi<DT>(tw[c]));
       }
+      if constexpr (EPI == GE_CONV) {
+        const uint32_t rw[4] = {rv[k].x, rv[k].y, rv[k].z, rv[k].w};
+        const float* f = &Fb[BN + q * 8];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          tw[c] = gm_pack2<DT>(gm_conv_tail_f<DT>(a, gm_lo<DT>(tw[c]), f[2 * c], f[BN + 2 * c], gm_lo<DT>(rw[c])),
+                               gm_conv_tail_f<DT>(a, gm_hi<DT>(tw[c]), f[2 * c + 1], f[BN + 2 * c + 1], gm_hi<DT>(rw[c])));
+      }
       *(uint4*)(OUT + (long long)m * a.ldo + n0) = make_uint4(tw[0], tw[1], tw[2], tw[3]);
     } else {   // rows that are no multiple of 16 bytes, or unaligned: one value at a time
 #pragma unroll
@@ -256,6 +319,9 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
         if (n0 + e >= N) continue;
         float v = (e & 1) ? gm_hi<DT>(tw[e >> 1]) : gm_lo<DT>(tw[e >> 1]);
         if constexpr (EPI == GE_RESID) v = gm_ld<DT>(a.resid, (long long)m * a.ldr + n0 + e) + v;
+        if constexpr (EPI == GE_CONV)
+          v = gm_conv_tail_f<DT>(a, v, Fb[BN + q * 8 + e], Fb[2 * BN + q * 8 + e],
+                                 (a.flags & 4) ? gm_ld<DT>(a.resid, (long long)m * a.ldr + n0 + e) : 0.f);
         OUT[(long long)m * a.ldo + n0 + e] = gm_pack<DT>(v);
       }
     }
@@ -293,3 +359,16 @@ TILE_KERNEL(k_gemm_bf16_silu_m256n144_w12_k64d, HS_BF16, GE_SILU, 2, 256, 144, 4
 TILE_GRP(k_gemm_bf16_grp_m64n64_k64d, HS_BF16, 64, 64, 4, 2, 8)
 TILE_GRP(k_gemm_bf16_grp_m64n128_k64d, HS_BF16, 64, 128, 2, 4, 6)
 TILE_GRP(k_gemm_bf16_grp_m128n128_k64d, HS_BF16, 128, 128, 2, 4, 4)
+// convolutions on channels-last activations with K > 1024 over many tiles (conv epilogue of gemm.hip): _conv reads the
+// [pixels, Cin] rows of the image (1 x 1, stride 1), _convg gathers 64 channels of one tap per stage
+#define TILE_CONV(DTN, DT, BM, BN, WR, WC, ST)                                                                          \
+  TILE_KERNEL(k_gemm_##DTN##_conv_m##BM##n##BN##_w8_k64d, DT, GE_CONV, 1, BM, BN, WR, WC, ST)                           \
+  extern "C" __global__ void __launch_bounds__(512) k_gemm_##DTN##_convg_m##BM##n##BN##_w8_k64d(const GemmArgs a) {     \
+    tile_body<DT, GE_CONV, 1, BM, BN, WR, WC, ST, false, true>(a);                                                      \
+  }
+TILE_CONV(f16, HS_F16, 64, 64, 4, 2, 8)
+TILE_CONV(f16, HS_F16, 64, 128, 2, 4, 6)
+TILE_CONV(f16, HS_F16, 128, 128, 2, 4, 4)
+TILE_CONV(bf16, HS_BF16, 64, 64, 4, 2, 8)
+TILE_CONV(bf16, HS_BF16, 64, 128, 2, 4, 6)
+TILE_CONV(bf16, HS_BF16, 128, 128, 2, 4, 4)

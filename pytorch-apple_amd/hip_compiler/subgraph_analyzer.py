@@ -61,6 +61,12 @@ WIDE_TA = 5
 WIDE_HALVES = os.environ.get("HIPRT_WIDE_HALVES", "1") == "1"
 GEMM_TARGET_WGS = 256    # workgroups a GEMM launch should reach (one per CU)
 GEMM_MIN_KCHUNK = 256    # smallest K range of one split-K workgroup
+# channels-last convs with longer K over at least this many 64 x 64 tiles run on tile.hip (ResNet-50 at
+# batch 32, 28 x 28 / 14 x 14 / 7 x 7 3 x 3: 23.0 / 26.8 / 26.4 -> 20.3 / 24.1 / 19.6 us). At shorter K a tile's few
+# stages go to its load latency and its stores, which more and smaller workgroups per CU overlap
+# better; at batch 1 (26 tiles) the one wide workgroup of a CU starts later (467 -> 473 us in all)
+CONV_TILE_MIN_K = 1024
+CONV_TILE_MIN_WGS = 128
 CONV_D2_MAX_K = int(os.environ.get("HIPRT_CONV_D2_MAX_K", "1024"))   # convs up to this K: 2-stage staging
 CONV_D1_MAX_K = int(os.environ.get("HIPRT_CONV_D1_MAX_K", "64"))   # emit_conv_nhwc: one-stage 64x64 kernels up to this K
 CONV_SMALL_TILE_MAX_K = 512   # conv_gemm_tiling: 64 x 64 tiles for K up to this over many tiles
@@ -76,6 +82,7 @@ TILE_COST = {
     "silu": {(64, 64, 8): (0.42, 1.4), (128, 144, 12): (1.0, 5.0), (256, 144, 12): (1.65, 8.0)},
     "one": {(64, 64, 8): (0.24, 2.1), (64, 96, 8): (0.31, 2.1), (128, 96, 8): (0.45, 1.5), (128, 128, 8): (0.495, 2.8),
             (256, 128, 8): (0.775, 4.9), (256, 256, 8): (1.55, 8.0)},
+    "conv": {(64, 64, 8): (0.35, 2.1), (64, 128, 8): (0.45, 2.8), (128, 128, 8): (0.66, 2.8)},   # tap gathers
     "grp": {(64, 64, 8): (0.24, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.495, 2.8)},
 }
 # us, us per byte of partials, per split (o_proj 128 x 1536 x 1536: 9.3 us with 4 splits, 9.9 with 5),
@@ -89,7 +96,7 @@ TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
 def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follows: bool = False) -> tuple[int, int, int, int]:
     """(BM, BN, waves, K splits) of the tile.hip kernel that TILE_COST expects to be fastest for an
     M x N x K GEMM, K % 64 == 0. ``kind``: "silu" (two weights), "one", or "grp" (columns of several
-    weights: BN divides every group boundary in ``bounds``); only "one" splits K.
+    weights: BN divides every group boundary in ``bounds``), "conv"; "one" and "conv" split K.
     ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
     (k_gemm_reduce_*_resid_norm), so it costs little more than its bytes. The line between
     two tiles lies where the rounds of workgroups make the smaller one cheaper: SiLU at N = 8960,
@@ -100,7 +107,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
         if any(b % bn for b in bounds):
             continue
         tiles = -(-M // bm) * -(-N // bn)
-        for ks in range(1, TILE_MAX_SPLIT + 1 if kind == "one" else 2):
+        for ks in range(1, TILE_MAX_SPLIT + 1 if kind in ("one", "conv") else 2):
             steps = -(-(K // 64) // ks)
             if ks > 1 and (steps * 64 < GEMM_MIN_KCHUNK or -(-(K // 64) // steps) != ks
                            or ks * M * N * 4 > TILE_MAX_PART or tiles * ks > 2 * TILE_CUS):
@@ -1185,11 +1192,17 @@ class Lowering:
         flags = (1 if has_bias else 0) | (2 if bn is not None else 0) | (4 if rv is not None else 0) | (8 if relu else 0)
         if CONV_NFAST and xv.numel > Cout * K:   # input larger than the weights: N tiles fastest
             flags |= 16
-        bm, bn_, ksplit = conv_gemm_tiling(M, Cout, K)
+        tile = K > CONV_TILE_MIN_K and -(-M // 64) * -(-Cout // 64) >= CONV_TILE_MIN_WGS
+        gn = 1
+        if tile:
+            bm, bn_, waves, ksplit = tile_plan(M, Cout, K, "conv")
+            gn = -(-Cout // bn_) if flags & 16 else tile_group(M, Cout, bm, bn_, 1, ksplit)
+        else:
+            bm, bn_, ksplit = conv_gemm_tiling(M, Cout, K)
         # always direct-to-LDS; K up to 1024 (at most 16 steps, where the pipeline depth buys little)
         # takes the 2-stage variant, whose smaller LDS footprint lets more workgroups share a CU
         # (the 56 x 56 3 x 3 convs, K = 576: 28 -> 25.5 us)
-        stages = "d2" if K <= CONV_D2_MAX_K else "d"
+        stages = "d2" if K <= CONV_D2_MAX_K or (bm, bn_) != (64, 64) else "d"
         if plain and K <= CONV_D1_MAX_K and (bm, bn_) == (64, 64) and ksplit == 1:
             stages = "d1"   # few K steps: one stage of LDS (16 KB), up to eight workgroups per CU
         kchunk = K
@@ -1199,7 +1212,7 @@ class Lowering:
         if self._conv_zero is None:
             self._conv_zero = self.scratch("conv.zero", 256, persistent=True)
         dts = "bf16" if dt == "bfloat16" else "f16"
-        kname = f"k_gemm_{dts}_{'conv' if plain else 'convg'}_m{bm}n{bn_}_k64{stages}"
+        kname = f"k_gemm_{dts}_{'conv' if plain else 'convg'}_m{bm}n{bn_}_" + (f"w{waves}_k64d" if tile else f"k64{stages}")
         part = self.scratch(out_name + ".kpart", ksplit * M * Cout * 4) if ksplit > 1 else None
         args = dict(x=self.ref(xv), w=self.ref(w), w2=None, bias=self.ref(self.contiguous(conv.inputs[2].name))
                     if has_bias else None, bias2=None, resid=self.ref(rv) if rv is not None else None,
@@ -1210,7 +1223,7 @@ class Lowering:
                     bn_mean=self.ref(bnv[2]) if bn is not None else None,
                     bn_var=self.ref(bnv[3]) if bn is not None else None,
                     zero=self._conv_zero, eps=float(bn.attrs.get("eps", 1e-5)) if bn is not None else 0.0,
-                    cH=H, cW=W, cCin=Cin, cHo=Ho, cWo=Wo, cKW=KW, csh=st[0], csw=st[1], cph=pd[0], cpw=pd[1])
+                    cH=H, cW=W, cCin=Cin, cHo=Ho, cWo=Wo, cKW=KW, csh=st[0], csw=st[1], cph=pd[0], cpw=pd[1], gn=gn)
         ins = [conv.inputs[0].name, wname] + ([conv.inputs[2].name] if has_bias else []) + \
             ([t.name for t in bn.inputs[1:5]] if bn is not None else []) + ([resid] if resid else [])
         params = {"M": M, "N": Cout, "K": K, "kernel": [KH, KW], "stride": st, "padding": pd,
@@ -1218,8 +1231,8 @@ class Lowering:
                   "ksplit": ksplit, "nhwc": True, "tile": (bm, bn_), "lds_direct": True, "stages": stages,
                   "nodes": nodes or [conv.name]}
         self.emit(LaunchStep(
-            kind="conv", kernel=kname, module="gemm", arg_struct="GemmArgs", args=args,
-            grid=((Cout + bn_ - 1) // bn_, (M + bm - 1) // bm, ksplit), inputs=ins,
+            kind="conv", kernel=kname, module="tile" if tile else "gemm", arg_struct="GemmArgs", args=args,
+            grid=((Cout + bn_ - 1) // bn_, (M + bm - 1) // bm, ksplit), block=(512 if tile else 256, 1, 1), inputs=ins,
             outputs=[out_name + ".kpart" if ksplit > 1 else out_name], params=params))
         if ksplit > 1:
             self.emit(LaunchStep(

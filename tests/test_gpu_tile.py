@@ -180,3 +180,72 @@ def test_silu_of_every_16_bit_value(backend):
     assert ((out[:, 0] - ref).abs() <= tol).all()
     exact = ref.bfloat16().double()
     assert ((out[:, 0] != exact) & (ref.abs() > 2.0 ** -121)).sum() <= 24   # 17 measured, as with expf and /
+
+
+@pytest.mark.parametrize("tile", [(64, 64, 8), (64, 128, 8), (128, 128, 8)])
+@pytest.mark.parametrize("N,H,W,C,Cout,k,stride,pad,add,dtype,ks", [
+    (1, 7, 7, 192, 96, 3, 1, 1, True, "float16", 1),      # 49 pixels, padded taps on every side, residual
+    (3, 9, 11, 128, 200, 3, 2, 1, False, "float16", 3),   # stride 2, odd sizes, ragged columns, split K
+    (2, 8, 9, 1088, 72, 1, 1, 0, True, "bfloat16", 1),    # the image rows as they are, 17 steps
+    (2, 13, 6, 1152, 68, 1, 2, 0, False, "float16", 2),   # strided 1 x 1; 68 columns: element-wise stores
+    (1, 6, 5, 128, 64, 5, 1, 2, False, "bfloat16", 1),    # 5 x 5: more padding than the image's half
+])
+def test_long_k_convolutions(backend, N, H, W, C, Cout, k, stride, pad, add, dtype, ks, tile, monkeypatch):
+    """Channels-last convs with K > 1024 (tile.hip's conv kernels) + batch norm (+ residual) + ReLU against
+    float64. Bound: with y the conv, v = r(r(y) a + b) (+ r): u |y| |a| + u |v| + u |out|, fp32 sums as above."""
+    import hip_compiler.subgraph_analyzer as SA
+    from irgen.builder import IRBuilder
+
+    monkeypatch.setattr(SA, "tile_plan", lambda M, n, K, kind, *a, **kw: tile + (ks,))
+    monkeypatch.setattr(SA, "CONV_TILE_MIN_WGS", 1)
+    td, u = (torch.float16, 2.0 ** -11) if dtype == "float16" else (torch.bfloat16, 2.0 ** -8)
+    g = torch.Generator(device="cuda").manual_seed(C + Cout)
+    rn = lambda *s, std=1.0, mean=0.0: (mean + std * torch.randn(s, generator=g, device="cuda")).to(td)
+    b = IRBuilder("conv")
+    x = b.input("x", [N, 64, H, W], dtype)
+    ident = b.weight("w0", [C, 64, 1, 1], dtype)   # a 1 x 1 that copies channels first: its output is channels-last
+    norm = lambda y, n, sfx: b.op("aten.batch_norm.default", [y] + [b.weight(q + sfx, [n], dtype) for q in (
+        "g", "beta", "mu", "var")], {"training": False, "momentum": 0.1, "eps": 1e-5, "cudnn_enabled": True})
+    h = b.op("aten.conv2d.default", [x, ident], {"stride": [1, 1], "padding": [0, 0], "dilation": [1, 1], "groups": 1})
+    h = b.op("aten.relu.default", [norm(h, C, "0")])   # (a factor of 1 / sqrt(1 + 1e-5): rounded away)
+    w = b.weight("w", [Cout, C, k, k], dtype)
+    y = b.op("aten.conv2d.default", [h, w], {"stride": [stride, stride], "padding": [pad, pad], "dilation": [1, 1],
+                                             "groups": 1})
+    y = norm(y, Cout, "")
+    if add:
+        y = b.op("aten.add.Tensor", [y, b.input("r", list(y.shape), dtype)])
+    b.output(b.op("aten.relu.default", [y]))
+    ir = b.to_dict()
+    K = C * k * k
+    pick = torch.arange(C) % 64
+    ws = {"w0": torch.eye(64, device="cuda")[pick.cuda()].reshape(C, 64, 1, 1).to(td), "w": rn(Cout, C, k, k, std=K ** -0.5),
+          "g": rn(Cout, std=0.1, mean=1.0), "beta": rn(Cout, std=0.1), "mu": rn(Cout, std=0.1),
+          "var": (torch.rand(Cout, generator=g, device="cuda") + 0.5).to(td)}
+    one, zero = torch.ones(C, dtype=td, device="cuda"), torch.zeros(C, dtype=td, device="cuda")
+    ws.update(g0=one, beta0=zero, mu0=zero, var0=one)
+    ins = {"x": rn(N, 64, H, W).abs()}
+    if add:
+        ins["r"] = rn(*[N, Cout, (H + 2 * pad - k) // stride + 1, (W + 2 * pad - k) // stride + 1])
+    print(f"[case] conv {N}x{C}x{H}x{W} -> {Cout} k{k} s{stride} p{pad} {dtype} tile {tile} ks {ks}", flush=True)
+    from hip_compiler import compile_subgraph, is_hip_op_supported
+    from npu_compiler import partition
+    from npu_runtime import DAGExecutor
+
+    ex = DAGExecutor(partition(ir, is_hip_op_supported), backend, compile_fn=compile_subgraph)
+    ex.load_weights(ws)
+    (out,) = ex.execute({n: backend.allocate_buffer(v) for n, v in ins.items()}).values()
+    (prog,) = ex.npu_programs.values()
+    main = [s for s in prog.steps if s.module == "tile" and s.params["kernel"] == [k, k] and s.args["N"] == Cout]
+    assert main and main[-1].kernel.endswith("_w8_k64d") and main[-1].args["ksplit"] == ks
+    d = {n: v.double().cpu() for n, v in {**ws, **ins}.items()}
+    d["x"] = d["x"][:, pick]
+    conv = lambda t, f: torch.nn.functional.conv2d(t, f, stride=stride, padding=pad)
+    yy, mag = conv(d["x"], d["w"]), conv(d["x"], d["w"].abs())
+    col = lambda t: t.reshape(1, -1, 1, 1)
+    a = d["g"] / torch.sqrt(d["var"] + 1e-5)
+    v = yy * col(a) + col(d["beta"] - d["mu"] * a)
+    ref = v + (d["r"] if add else 0.0)
+    s32 = K * 2.0 ** -24 * (mag + 1.0)
+    tol = 1.02 * (u * (yy.abs() * col(a).abs() + v.abs() + ref.abs()) + s32 * (1 + col(a).abs())) + 1e-6
+    bad = (out.to_torch().cpu().double() - ref.clamp(min=0)).abs() > tol
+    assert not bad.any(), (int(bad.sum()), bad.nonzero()[0].tolist())
