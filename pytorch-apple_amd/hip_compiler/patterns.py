@@ -33,6 +33,8 @@ FUSE_REDUCE_NORM = True
 # each, 18.6 with three; 2000 tokens 51 with three, in 252 workgroups)
 PREFILL_ATTN_WGS = 256
 
+ROPE_SLOTS = 4   # heads per wave of k_rope_cache (RC_SLOTS in gemv.hip)
+
 _PASS = ("aten._assert_tensor_metadata.default",)
 
 
@@ -933,7 +935,7 @@ def _emit_qkv_prefill(low, xname, q, k, v, names) -> None:
                  cpos_dtype=DTYPE_CODE[cpos.dtype], dtype=DTYPE_CODE["bfloat16"],
                  rope_scaling=float(rope.attrs.get("attention_scaling", 1.0)))
     low.emit(LaunchStep(kind="gemv", kernel="k_rope_cache", module="gemv", arg_struct="RopeCacheArgs", args=rargs,
-                        grid=((T * (H + 2 * KVH) + 3) // 4, 1, 1), inputs=[y.storage, k["cpos"], k["past"], v["past"]],
+                        grid=((T * -(-(H + 2 * KVH) // ROPE_SLOTS) + 3) // 4, 1, 1), inputs=[y.storage, k["cpos"], k["past"], v["past"]],
                         outputs=[q["out"], k["ic"].outputs[0].name, v["ic"].outputs[0].name],
                         params={"T": T, "heads": [H, KVH], "nodes": names}))
     low.views[q["out"]] = qo
