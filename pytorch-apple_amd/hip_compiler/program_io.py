@@ -83,7 +83,16 @@ def program_from_dict(data: dict) -> HIPProgram:
     names = {f.name for f in dataclasses.fields(HIPProgram)}
     if set(body) != names:
         raise ValueError(f"program fields differ: {sorted(set(body) ^ names)}")
-    return HIPProgram(**{k: _dec(v) for k, v in body.items()})
+    prog = HIPProgram(**{k: _dec(v) for k, v in body.items()})
+    # k_mask_extent writes two ints per 32-query block; files written when it wrote one hold half the bytes
+    for step in prog.steps:
+        if step.kernel == "k_mask_extent":
+            need = 8 * ((step.args["T"] + 31) // 32)
+            ref = step.args["nblk_out"]
+            if ref.byte_offset + need > prog.storages[ref.storage].nbytes:
+                raise ValueError(f"mask extents of {need} bytes do not fit storage {ref.storage!r}: the program was "
+                                 "compiled for other kernels, compile it again")
+    return prog
 
 
 def save_program(prog: HIPProgram, path: str) -> None:

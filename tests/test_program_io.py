@@ -44,6 +44,17 @@ def test_hipbin_rejects_other_formats_and_unknown_records(tmp_path):
         program_from_dict(bad)
 
 
+def test_hipbin_with_smaller_mask_extents_is_refused():
+    """A file from before the mask-extent kernel wrote two ints per query block would be written past."""
+    d = json.loads(json.dumps(program_to_dict(compile_subgraph(graphs()["prefill"]))))
+    program_from_dict(d)
+    ext = [s for s in d["program"]["storages"].values() if ".extent" in s["name"]]
+    assert ext
+    ext[0]["nbytes"] //= 2
+    with pytest.raises(ValueError, match="compile it again"):
+        program_from_dict(d)
+
+
 def test_program_cache_hits_and_keys(tmp_path):
     ir = graphs()["decode"]
     a = compile_cached(ir, str(tmp_path))
