@@ -812,7 +812,8 @@ GEMM_KERNEL_K64(k_gemm_f16_bias_m64n64, HS_F16, GE_BIAS, 1, 64, 64)
   extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_convp_m##BM##n##BN##_k64d2(const GemmArgs a) {            \
     gemm_body<DT, GE_CONV, 1, BM, BN, false, 64, false, 2, 2>(a);                                                   \
   }
-// long K over few tiles (the wide tiles of long K run on tile.hip): four stages
+// four stages: long K over few tiles (the wide tiles of long K run on tile.hip), and 1 x 1 convs of any K with
+// a CU to each workgroup, where nothing else hides a step's load latency (ResNet-50 at batch 1: 467 -> 450 us)
 #define GEMM_CONV_D(DTN, DT)                                                                                        \
   extern "C" __global__ void GM_ATTRS_CONV k_gemm_##DTN##_conv_m64n64_k64d(const GemmArgs a) {                      \
     gemm_body<DT, GE_CONV, 1, 64, 64, false, 64, false, 4>(a);                                                      \

@@ -140,6 +140,11 @@ def lowering_settings(options: dict) -> dict:
         "conv_d2_max_k": subgraph_analyzer.CONV_D2_MAX_K,
         "conv_small_tile_max_k": subgraph_analyzer.CONV_SMALL_TILE_MAX_K,
         "conv_nfast": bool(subgraph_analyzer.CONV_NFAST),
+        "conv_d_wgs": int(subgraph_analyzer.CONV_D_WGS),
+        "conv_split_short_tiles": int(subgraph_analyzer.CONV_SPLIT_SHORT_TILES),
+        "conv_tile_min_k": int(subgraph_analyzer.CONV_TILE_MIN_K),
+        "conv_tile_min_wgs": int(subgraph_analyzer.CONV_TILE_MIN_WGS),
+        "prefill_attn_wgs": int(patterns.PREFILL_ATTN_WGS),
         "conv_d1_max_k": subgraph_analyzer.CONV_D1_MAX_K,
         "fuse_reduce_norm": bool(patterns.FUSE_REDUCE_NORM),
         "persistent_decode": (os.environ.get("HIPRT_PERSISTENT", "1") == "1") if options.get("persistent") is None

@@ -68,6 +68,15 @@ GEMM_MIN_KCHUNK = 256    # smallest K range of one split-K workgroup
 CONV_TILE_MIN_K = 1024
 CONV_TILE_MIN_WGS = 128
 CONV_D2_MAX_K = int(os.environ.get("HIPRT_CONV_D2_MAX_K", "1024"))   # convs up to this K: 2-stage staging
+# 1 x 1 convs of at most this many 64 x 64 workgroups (one per CU: nothing else shares its LDS) keep four
+# stages in flight instead of two at any K (ResNet-50 at batch 1 / 2 / 5: 467 / 487 / 572 -> 450 / 471 / 558 us;
+# 512 workgroups: within 1% of 256). Gathered taps of short K stay on two stages, as test_gpu_parity.py asks (with
+# four: another 5, 4 and 4 us)
+CONV_D_WGS = 256
+# convs of K = 1024 .. 2047 split K only below this many 64 x 64 tiles: a split saves at most 12-24 steps of
+# 0.4 us, and its reduce costs 4 us and the partials' bytes (ResNet-50 without / with: batch 2 466 / 474 us at 28
+# tiles of K = 1024, batch 5 544 / 555 and batch 8 619 / 646 at 64 and 100)
+CONV_SPLIT_SHORT_TILES = 64
 CONV_D1_MAX_K = int(os.environ.get("HIPRT_CONV_D1_MAX_K", "64"))   # emit_conv_nhwc: one-stage 64x64 kernels up to this K
 CONV_SMALL_TILE_MAX_K = 512   # conv_gemm_tiling: 64 x 64 tiles for K up to this over many tiles
 CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order by operand sizes (emit_conv_nhwc)
@@ -168,8 +177,9 @@ def conv_gemm_tiling(M: int, N: int, K: int) -> tuple[int, int, int]:
     """(BM, BN, split-K) for a conv as a GEMM over M pixels, N output channels, K = KH*KW*Cin:
     64 x 64 for short K over many tiles (K <= 512, >= 1024 tiles); otherwise the largest tile no
     wider than the channels that still gives >= 256 workgroups; smaller
-    grids take 64 x 64 tiles and, for K >= 1024, split K toward ~384 workgroups (fp32
-    partials, then the reduce applies the epilogue)."""
+    grids take 64 x 64 tiles and, for K >= 2048, or K >= 1024 over few tiles
+    (CONV_SPLIT_SHORT_TILES), split K toward ~384 workgroups (fp32 partials, then the reduce
+    applies the epilogue)."""
     ntiles = lambda bm, bn: ((M + bm - 1) // bm) * ((N + bn - 1) // bn)
     if K <= CONV_SMALL_TILE_MAX_K and ntiles(64, 64) >= 4 * GEMM_TARGET_WGS:
         # short K, many tiles: the time goes to each tile's load latency and store drain, not to
@@ -181,7 +191,7 @@ def conv_gemm_tiling(M: int, N: int, K: int) -> tuple[int, int, int]:
         if ntiles(bm, bn) >= GEMM_TARGET_WGS:
             return bm, bn, 1
     t = ntiles(64, 64)
-    if K >= 1024:
+    if K >= 2048 or (K >= 1024 and t < CONV_SPLIT_SHORT_TILES):
         return 64, 64, max(1, min(8, (384 + t - 1) // t, K // GEMM_MIN_KCHUNK))
     return 64, 64, 1
 
@@ -1203,6 +1213,8 @@ class Lowering:
         # takes the 2-stage variant, whose smaller LDS footprint lets more workgroups share a CU
         # (the 56 x 56 3 x 3 convs, K = 576: 28 -> 25.5 us)
         stages = "d2" if K <= CONV_D2_MAX_K or (bm, bn_) != (64, 64) else "d"
+        if plain and (bm, bn_) == (64, 64) and -(-M // 64) * -(-Cout // 64) * ksplit <= CONV_D_WGS:
+            stages = "d"   # a CU to itself: the loads in flight count, not the footprint
         if plain and K <= CONV_D1_MAX_K and (bm, bn_) == (64, 64) and ksplit == 1:
             stages = "d1"   # few K steps: one stage of LDS (16 KB), up to eight workgroups per CU
         kchunk = K
