@@ -742,9 +742,9 @@ PA_KERNEL(k_attn_prefill_f16_f32mask, HS_F16, 2)
 // not read), 0 when there is none. Every block past it is closed for all of those rows, so
 // k_attn_prefill leaves it out: its terms would be e^-inf = 0 exactly. NaN entries count as
 // open. nblk_out[2 qb + 1] = c / 32 for the smallest column c whose entry is not (+-)0 in some row
-// (S / 32 when there is none): the blocks below it add nothing to any score. Wave w scans rows w and w + 16, lanes along the row, all loads of a 2048-column chunk
-// (eight per lane) issued before the first is tested, so a scan of S <= 2048 is one memory
-// latency. 16-bit masks are read four entries per 8-byte load (unit column stride, 8-byte aligned
+// (S / 32 when there is none): the blocks below it add nothing to any score. Wave w scans rows w and
+// w + 16, lanes along the row, all loads of a 2048-column chunk (eight per lane) issued before the
+// first is tested, so a scan of S <= 2048 is one memory latency. 16-bit masks are read four entries per 8-byte load (unit column stride, 8-byte aligned
 // rows, S % 4 == 0: the host checks).
 extern "C" __global__ void __launch_bounds__(1024) k_mask_extent(const MaskExtentArgs a) {
   __shared__ int best[16], first[16];

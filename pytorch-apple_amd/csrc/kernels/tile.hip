@@ -29,9 +29,9 @@
 //   BIAS  out = round(acc + b)
 //   RESID out = round(r + round(acc + b))
 //   SILU  out = round(round(silu(round(acc_g + b_g))) * round(acc_u + b_u))   (NW = 2)
+//   CONV  round(acc + b), batch norm, residual and ReLU as gemm.hip's conv epilogue
 // ksplit > 1: grid.z workgroups take kchunk of K each and store fp32 partials [z, NW, M, N]; a
 // k_gemm_reduce_* kernel (gemm.hip) sums them in order and applies the epilogue.
-//   CONV  round(acc + b), batch norm, residual and ReLU as gemm.hip's conv epilogue
 // CV: x rows are gathered from an NHWC image, one tap and 64 channels per stage (K = (kh, kw, ci),
 // cCin % 64 == 0), taps outside it from a.zero. ResNet-50's 3 x 3 convs at batch 32 with 128 / 256 / 512
 // channels: 23.0 / 26.8 / 26.4 -> 20.3 / 24.1 / 19.6 us against the 4-wave kernels; they take in 45-60 GB/s

@@ -29,8 +29,7 @@ from npu_compiler.ir_reader import OpNode
 FUSE_REDUCE_NORM = True
 
 # workgroups of prefill attention up to which a workgroup takes fewer heads (one per CU; 512 tokens of
-# 12 heads 13.5 us with one head
-# each, 18.6 with three; 2000 tokens 51 with three, in 252 workgroups)
+# 12 heads 13.5 us with one head each, 18.6 with three; 2000 tokens 51 with three, in 252 workgroups)
 PREFILL_ATTN_WGS = 256
 
 ROPE_SLOTS = 4   # heads per wave of k_rope_cache (RC_SLOTS in gemv.hip)
