@@ -45,6 +45,12 @@ def _mask(kind, T, S):
     elif kind == "lowest":
         m[s > t] = torch.finfo(torch.bfloat16).min
         m[T // 2] = torch.finfo(torch.bfloat16).min
+    elif kind == "bias":    # values in every open block
+        m = -(t + (S - T) - s).clamp(min=0) / 64
+        m[s > t + (S - T)] = -torch.inf
+    elif kind == "mixed":   # open blocks, then values, then closed blocks, then values to the end
+        m = torch.cos(0.37 * s + t) * (s >= 170)
+        m[:, 400:520] = -torch.inf
     return m
 
 
@@ -60,6 +66,10 @@ def _mask(kind, T, S):
     (50, 132, 12, 2, "bfloat16", "bfloat16", "lowest"),
     (66, 260, 12, 2, "float16", "float16", "causal"),
     (34, 96, 4, 2, "float16", None, "open"),
+    (45, 700, 12, 2, "bfloat16", "bfloat16", "bias"),      # mask values over several rounds of blocks
+    (33, 644, 6, 1, "bfloat16", "bfloat16", "mixed"),
+    (33, 644, 4, 2, "bfloat16", "float32", "mixed"),
+    (40, 388, 12, 2, "float16", "float16", "mixed"),
 ])
 @pytest.mark.parametrize("heads", [1, 2, 3])
 def test_prefill_attention_vs_float64(backend, T, S, H, KVH, dtype, mask_dtype, kind, heads, monkeypatch):
