@@ -1,6 +1,6 @@
 // MFMA GEMM on wide workgroups: out[m, n] = epi(sum_k x[m, k] w[n, k]) for activations [M, K] and
-// weights [N, K] as the model stores them, K % 64 == 0. One workgroup of WR x WC waves (8 or 12) per
-// CU and BM x BN output tile.
+// weights [N, K] as the model stores them, K % 64 == 0. One workgroup of WR x WC waves (8, 10 or 12)
+// per BM x BN output tile, and per CU (two with 64 x 64 tiles).
 //
 // What bounds a GEMM of these shapes (M = 128 .. 4096 against 1536- to 151936-row weights) is how
 // many operand bytes a CU has in flight and takes in per MFMA, not the MFMA rate itself. So:
@@ -8,21 +8,27 @@
 //     filled by global_load_lds_dwordx4 (128-byte rows, whole cache lines; 64-byte rows, twice as
 //     many stages of half the depth, were 10-15% slower: each line is then fetched twice);
 //   * tiles are as large as the shape allows while the grid still fills the 256 CUs in whole
-//     rounds (the host's tile_plan): 256 x 144 of both SiLU weights is 252 workgroups at M = 1000;
+//     rounds (the host's tile_plan): 256 x 144 of both SiLU weights is 252 workgroups at M = 1000,
+//     192 x 144 is 252 at 768 (45 us; 128 x 144 48), 128 x 80 224 at 256 (24 us; 128 x 144 33);
+//   * 64 x 64 tiles take half the LDS (rings of 4 stages, 3 with two weights), so that two workgroups
+//     share a CU and 257 to 512 of them are one round: o_proj (N = K = 1536) at M = 1025 14.2 us on
+//     128 x 96 tiles, 18.0 on 64 x 64 with the whole LDS, 12.0 now; no slower where one has a CU to itself;
 //   * each operand address is a scalar base plus a 32-bit lane offset (one SALU add per load);
-//   * 12 waves (three per SIMD) on the tiles whose widths are 3 x 96 or 3 x 48, 8 on the others; the
+//   * 12 waves (three per SIMD) on the tiles of width 3 x 48, 10 on those of 5 x 16, 8 on the others; the
 //     16-byte chunks of a row sit in slot c ^ ((row >> 1) & 7), which the 16 x 4 fragment reads of
 //     v_mfma_f32_16x16x32 cross without a bank conflict (237 bytes per clock and CU measured; 63 with
 //     the chunks in order).
 // The MFMA computes the transposed tile (weights as operand A), so that a lane holds 4 consecutive
 // columns of one row: 8-byte LDS writes in the epilogue, 16-byte rows out of it, and float4 partials.
 //
-// Measured on MI355X (bf16, kernel alone, weights rotated through 4 copies), against the 4-wave
-// kernels of gemm.hip: gate/up with SiLU (N = 8960, K = 1536) at M = 512 / 1000 / 2000
-// 47 / 75 / 142 -> 32 / 50 / 97 us; lm_head 512 x 151936 x 1536 325 -> 234 us (1,020 TFLOP/s);
-// down_proj (N = 1536, K = 8960) at M = 512, 5 K splits, 26 -> 20 us, at 1000 60 -> 32 us plus the
-// reduce. A steady K step of 256 x 256 takes 1.56 us (1,376 TFLOP/s over 256 CUs); a launch spends
-// the rest (8-11 us) on its first stage's latency and its epilogue.
+// Measured on MI355X (bf16, calls of one launch or of one and its reduce, as many copies of the weights as
+// come from HBM), against the 4-wave kernels of gemm.hip that ran these before: gate/up with SiLU (N = 8960,
+// K = 1536) at M = 192 / 512 / 1000 / 2000 27 / 46 / 75 / 133 -> 23 / 35 / 53 / 103 us; lm_head
+// (N = 151936, K = 1536) at M = 513 373 -> 321 us; down_proj (N = 1536, K = 8960) at M = 512 / 1000 / 2000
+// 35 / 75 / 99 -> 28 / 42 / 68 us. The slowest rounds left: gate/up at M = 1090 .. 1152, 378 tiles of 192 x 144
+// in two rounds, is where the 4-wave kernels' 846 tiles were (83-84 us both). A steady K step of
+// 256 x 256 takes 1.56 us (1,376 TFLOP/s over 256 CUs); a launch spends the rest (8-11 us) on its first
+// stage's latency and its epilogue.
 //
 // Epilogues (fp32 accumulator, ATen's rounding points), rows past M and columns past N clamped when
 // read and not stored:
@@ -339,7 +345,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
     tile_body<DT, GE_BIAS, 1, BM, BN, WR, WC, ST, true>(a);                                       \
   }
 #define TILE_BIAS(DTN, DT)                                                                        \
-  TILE_KERNEL(k_gemm_##DTN##_bias_m64n64_w8_k64d, DT, GE_BIAS, 1, 64, 64, 4, 2, 8)                \
+  TILE_KERNEL(k_gemm_##DTN##_bias_m64n64_w8_k64d, DT, GE_BIAS, 1, 64, 64, 4, 2, 4)                \
   TILE_KERNEL(k_gemm_##DTN##_bias_m64n96_w8_k64d, DT, GE_BIAS, 1, 64, 96, 4, 2, 6)                \
   TILE_KERNEL(k_gemm_##DTN##_bias_m128n96_w8_k64d, DT, GE_BIAS, 1, 128, 96, 4, 2, 5)              \
   TILE_KERNEL(k_gemm_##DTN##_bias_m128n128_w8_k64d, DT, GE_BIAS, 1, 128, 128, 2, 4, 4)            \
@@ -347,16 +353,18 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   TILE_KERNEL(k_gemm_##DTN##_bias_m256n256_w8_k64d, DT, GE_BIAS, 1, 256, 256, 2, 4, 2)
 TILE_BIAS(bf16, HS_BF16)
 TILE_BIAS(f16, HS_F16)
-TILE_KERNEL(k_gemm_bf16_resid_m64n64_w8_k64d, HS_BF16, GE_RESID, 1, 64, 64, 4, 2, 8)
+TILE_KERNEL(k_gemm_bf16_resid_m64n64_w8_k64d, HS_BF16, GE_RESID, 1, 64, 64, 4, 2, 4)
 TILE_KERNEL(k_gemm_bf16_resid_m64n96_w8_k64d, HS_BF16, GE_RESID, 1, 64, 96, 4, 2, 6)
 TILE_KERNEL(k_gemm_bf16_resid_m128n96_w8_k64d, HS_BF16, GE_RESID, 1, 128, 96, 4, 2, 5)
 TILE_KERNEL(k_gemm_bf16_resid_m128n128_w8_k64d, HS_BF16, GE_RESID, 1, 128, 128, 2, 4, 4)
 TILE_KERNEL(k_gemm_bf16_resid_m256n128_w8_k64d, HS_BF16, GE_RESID, 1, 256, 128, 4, 2, 3)
 TILE_KERNEL(k_gemm_bf16_resid_m256n256_w8_k64d, HS_BF16, GE_RESID, 1, 256, 256, 2, 4, 2)
-TILE_KERNEL(k_gemm_bf16_silu_m64n64_w8_k64d, HS_BF16, GE_SILU, 2, 64, 64, 2, 4, 6)
+TILE_KERNEL(k_gemm_bf16_silu_m64n64_w8_k64d, HS_BF16, GE_SILU, 2, 64, 64, 2, 4, 3)
+TILE_KERNEL(k_gemm_bf16_silu_m128n80_w10_k64d, HS_BF16, GE_SILU, 2, 128, 80, 2, 5, 4)
 TILE_KERNEL(k_gemm_bf16_silu_m128n144_w12_k64d, HS_BF16, GE_SILU, 2, 128, 144, 4, 3, 3)
+TILE_KERNEL(k_gemm_bf16_silu_m192n144_w12_k64d, HS_BF16, GE_SILU, 2, 192, 144, 4, 3, 2)
 TILE_KERNEL(k_gemm_bf16_silu_m256n144_w12_k64d, HS_BF16, GE_SILU, 2, 256, 144, 4, 3, 2)
-TILE_GRP(k_gemm_bf16_grp_m64n64_k64d, HS_BF16, 64, 64, 4, 2, 8)
+TILE_GRP(k_gemm_bf16_grp_m64n64_k64d, HS_BF16, 64, 64, 4, 2, 4)
 TILE_GRP(k_gemm_bf16_grp_m64n128_k64d, HS_BF16, 64, 128, 2, 4, 6)
 TILE_GRP(k_gemm_bf16_grp_m128n128_k64d, HS_BF16, 128, 128, 2, 4, 4)
 // convolutions on channels-last activations with K > 1024 over many tiles (conv epilogue of gemm.hip): _conv reads the
@@ -366,9 +374,9 @@ TILE_GRP(k_gemm_bf16_grp_m128n128_k64d, HS_BF16, 128, 128, 2, 4, 4)
   extern "C" __global__ void __launch_bounds__(512) k_gemm_##DTN##_convg_m##BM##n##BN##_w8_k64d(const GemmArgs a) {     \
     tile_body<DT, GE_CONV, 1, BM, BN, WR, WC, ST, false, true>(a);                                                      \
   }
-TILE_CONV(f16, HS_F16, 64, 64, 4, 2, 8)
+TILE_CONV(f16, HS_F16, 64, 64, 4, 2, 4)
 TILE_CONV(f16, HS_F16, 64, 128, 2, 4, 6)
 TILE_CONV(f16, HS_F16, 128, 128, 2, 4, 4)
-TILE_CONV(bf16, HS_BF16, 64, 64, 4, 2, 8)
+TILE_CONV(bf16, HS_BF16, 64, 64, 4, 2, 4)
 TILE_CONV(bf16, HS_BF16, 64, 128, 2, 4, 6)
 TILE_CONV(bf16, HS_BF16, 128, 128, 2, 4, 4)

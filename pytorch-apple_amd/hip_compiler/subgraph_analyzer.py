@@ -82,17 +82,21 @@ CONV_SMALL_TILE_MAX_K = 512   # conv_gemm_tiling: 64 x 64 tiles for K up to this
 CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order by operand sizes (emit_conv_nhwc)
 
 
-# tile.hip kernels: (BM, BN, waves) -> (us per K step of 64, us per round of workgroups), by the kind
-# of launch. Fitted on MI355X to the kernels alone over M = 40 .. 4096 against weights of 1536 x 8960,
-# 1536 x 1536, 2048 x 1536, 4096 x 1536, 8960 x 1536 (SiLU pairs) and 151936 x 1536: a launch takes
-# ceil(workgroups / 256) rounds of (K / 64 steps + fixed), 2 us, and with K split TILE_REDUCE: the
-# reduce's 4 us and 0.2 us per MB of fp32 partials; within 10% of what was measured at all of them.
+# tile.hip kernels: (BM, BN, waves) -> (us per K step of 64, us per round of workgroups[, us per K step when
+# two workgroups share a CU]), by the kind of launch. Fitted on MI355X to calls over M = 33 .. 4096 against
+# weights of 1536 x 8960, 1536 x 1536, 4096 x 4096, 2560 x 2048, 512 x 512 (one weight, 1 to 16 K splits) and
+# 8960 x 1536, 4864 x 896, 11008 x 4096, 1024 x 512 (SiLU pairs), enough copies of them that they come from HBM:
+# a call takes 2 us and ceil(workgroups / (CUs x workgroups per CU)) rounds of (K / 64 steps + fixed), with K
+# split also TILE_REDUCE. Of the plans measured within 25% of a size's fastest that is 7% off (rms; 20% low to
+# 29% high), and the plan it picks is 0.5% slower than the fastest on average, 11% at worst (SiLU at
+# 3000 x 1024 x 512). Launches inside a layer, with other kernels before them, take 5-20% longer.
 TILE_COST = {
-    "silu": {(64, 64, 8): (0.42, 1.4), (128, 144, 12): (1.0, 5.0), (256, 144, 12): (1.65, 8.0)},
-    "one": {(64, 64, 8): (0.24, 2.1), (64, 96, 8): (0.31, 2.1), (128, 96, 8): (0.45, 1.5), (128, 128, 8): (0.495, 2.8),
-            (256, 128, 8): (0.775, 4.9), (256, 256, 8): (1.55, 8.0)},
-    "conv": {(64, 64, 8): (0.35, 2.1), (64, 128, 8): (0.45, 2.8), (128, 128, 8): (0.66, 2.8)},   # tap gathers
-    "grp": {(64, 64, 8): (0.24, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.495, 2.8)},
+    "silu": {(64, 64, 8): (0.4, 1.5, 0.8), (128, 80, 10): (0.68, 3.1), (128, 144, 12): (1.02, 3.75),
+             (192, 144, 12): (1.39, 4.75), (256, 144, 12): (1.64, 5.5)},
+    "one": {(64, 64, 8): (0.2, 2.2, 0.39), (64, 96, 8): (0.32, 1.6), (128, 96, 8): (0.46, 1.7), (128, 128, 8): (0.535, 2.6),
+            (256, 128, 8): (0.82, 3.8), (256, 256, 8): (1.45, 7.0)},
+    "conv": {(64, 64, 8): (0.35, 2.1, 0.55), (64, 128, 8): (0.45, 2.8), (128, 128, 8): (0.66, 2.8)},   # tap gathers
+    "grp": {(64, 64, 8): (0.21, 2.1, 0.36), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.5, 2.6)},
 }
 # us, us per byte of partials, per split (o_proj 128 x 1536 x 1536: 9.3 us with 4 splits, 9.9 with 5),
 # and for a second round of 8 splits' loads
@@ -102,17 +106,30 @@ TILE_MAX_SPLIT = 16
 TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
 
 
+def tile_us(kind: str, tile: tuple, wgs: int, steps: int) -> float:
+    """us that TILE_COST gives ``wgs`` workgroups of ``steps`` K steps each."""
+    step, fixed, *shared = TILE_COST[kind][tile]
+    if not shared:
+        return -(-wgs // TILE_CUS) * (steps * step + fixed)
+    full, rest = divmod(wgs, 2 * TILE_CUS)
+    last = 0.0 if not rest else steps * (shared[0] if rest > TILE_CUS else step) + fixed
+    return full * (steps * shared[0] + fixed) + last
+
+
 def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follows: bool = False) -> tuple[int, int, int, int]:
     """(BM, BN, waves, K splits) of the tile.hip kernel that TILE_COST expects to be fastest for an
     M x N x K GEMM, K % 64 == 0. ``kind``: "silu" (two weights), "one", or "grp" (columns of several
     weights: BN divides every group boundary in ``bounds``), "conv"; "one" and "conv" split K.
     ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
     (k_gemm_reduce_*_resid_norm), so it costs little more than its bytes. The line between
-    two tiles lies where the rounds of workgroups make the smaller one cheaper: SiLU at N = 8960,
-    K = 1536 takes 128 x 144 tiles up to M = 512 (252 workgroups, 32 us; 256 x 144 43) and
-    256 x 144 at 1000 (252 workgroups, 50 us; 128 x 144 60)."""
+    two tiles lies where the rounds of workgroups make the smaller one cheaper. SiLU at N = 8960,
+    K = 1536: 128 x 80 tiles up to M = 256 (224 workgroups, 24 us; 128 x 144 33), 128 x 144 up to 512 (252, 34 us;
+    192 x 144 44), 192 x 144 up to 768 (252, 45 us; 128 x 144 48, 256 x 144 51) and again at 1025 .. 1536
+    (378 to 504 workgroups, 81-86 us; 128 x 144 85-95), 256 x 144 at 769 .. 1024 (252, 51 us; 128 x 144 60)
+    and at 1537 .. 2048 (504, 93-100). 64 x 64 tiles run two workgroups per CU: o_proj (N = K = 1536) at
+    M = 1025 .. 1152 is one round of 408 to 432, 12.0-12.4 us against 14.2 on 128 x 96."""
     best = None
-    for (bm, bn, waves), (step, fixed) in TILE_COST[kind].items():
+    for bm, bn, waves in TILE_COST[kind]:
         if any(b % bn for b in bounds):
             continue
         tiles = -(-M // bm) * -(-N // bn)
@@ -121,7 +138,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
             if ks > 1 and (steps * 64 < GEMM_MIN_KCHUNK or -(-(K // 64) // steps) != ks
                            or ks * M * N * 4 > TILE_MAX_PART or tiles * ks > 2 * TILE_CUS):
                 continue
-            us = -(-tiles * ks // TILE_CUS) * (steps * step + fixed)
+            us = tile_us(kind, (bm, bn, waves), tiles * ks, steps)
             if ks > 1:
                 us += (1.5 if norm_follows else TILE_REDUCE[0]) + TILE_REDUCE[1] * ks * M * N * 4
                 us += TILE_REDUCE[2] * ks + (TILE_REDUCE[3] if ks > 8 else 0.0)

@@ -35,3 +35,31 @@ def test_plan_covers_the_product(kind, bounds):
                 assert ks == 1 or (kind == "one" and (ks - 1) * chunk < K <= ks * chunk and chunk >= GEMM_MIN_KCHUNK
                                    and ks * M * N * 4 <= TILE_MAX_PART)
                 assert 1 <= tile_group(M, N, bm, bn, 2 if kind == "silu" else 1, ks) <= -(-N // bn)
+
+
+@pytest.mark.parametrize("kind,N,K,rows,tile", [
+    ("silu", 8960, 1536, (129, 160, 192, 256), (128, 80)),       # on 64 x 64, one per CU, 420 tiles were two rounds
+    ("silu", 8960, 1536, (513, 640, 768), (192, 144)),
+    ("silu", 8960, 1536, (1025, 1088, 1152, 1280), (192, 144)),  # on 128 x 144 three rounds
+    ("one", 1536, 1536, (1025, 1152, 1281), (64, 64)),           # two per CU: one round of half-size workgroups
+])
+def test_rows_just_past_a_full_round(kind, N, K, rows, tile):
+    """Row counts just past a full round of the larger tiles take tiles that fill the CUs again, not a
+    nearly empty last round of the larger ones."""
+    from hip_compiler.subgraph_analyzer import tile_plan
+
+    for M in rows:
+        assert tile_plan(M, N, K, kind)[:2] == tile, M
+
+
+def test_two_workgroups_per_cu_are_one_round():
+    """The third number of a TILE_COST entry: 257 to 512 workgroups are one round of shared CUs, and what is
+    left of a round goes at the rate of a CU to each."""
+    from hip_compiler.subgraph_analyzer import TILE_COST, tile_us
+
+    tile = (64, 64, 8)
+    step, fixed, shared = TILE_COST["one"][tile]
+    for wgs, us in ((1, step), (256, step), (257, shared), (512, shared)):
+        assert tile_us("one", tile, wgs, 10) == pytest.approx(10 * us + fixed)
+    assert tile_us("one", tile, 600, 10) == pytest.approx(10 * (shared + step) + 2 * fixed)
+    assert tile_us("one", (128, 128, 8), 257, 10) == pytest.approx(2 * tile_us("one", (128, 128, 8), 256, 10))
