@@ -67,6 +67,10 @@ GEMM_MIN_KCHUNK = 256    # smallest K range of one split-K workgroup
 # better; at batch 1 (26 tiles) the one wide workgroup of a CU starts later (467 -> 473 us in all)
 CONV_TILE_MIN_K = 1024
 CONV_TILE_MIN_WGS = 128
+# up to 64 output channels only within one round of 64 x 64 tiles: past it the wider tiles' empty columns cost more
+# than they save, and the 4-wave kernels' 128 x 64 tiles have none (3 x 3, 128 -> 64, with the conv before it: 10 images
+# of 56 x 56, 490 tiles, 45 us on tile.hip; 11, 539 tiles, 62 on tile.hip, 51 on 4 waves; 64, 219 and 160)
+CONV_TILE_NARROW_WGS = 512
 CONV_D2_MAX_K = int(os.environ.get("HIPRT_CONV_D2_MAX_K", "1024"))   # convs up to this K: 2-stage staging
 # 1 x 1 convs of at most this many 64 x 64 workgroups (one per CU: nothing else shares its LDS) keep four
 # stages in flight instead of two at any K (ResNet-50 at batch 1 / 2 / 5: 467 / 487 / 572 -> 450 / 471 / 558 us;
@@ -82,8 +86,8 @@ CONV_SMALL_TILE_MAX_K = 512   # conv_gemm_tiling: 64 x 64 tiles for K up to this
 CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order by operand sizes (emit_conv_nhwc)
 
 
-# tile.hip kernels: (BM, BN, waves) -> (us per K step of 64, us per round of workgroups[, us per K step when
-# two workgroups share a CU]), by the kind of launch. Fitted on MI355X to calls over M = 33 .. 4096 against
+# tile.hip kernels: (BM, BN, waves) -> (us per K step of 64, us per round of workgroups[, the same when two
+# workgroups share a CU]), by the kind of launch. Fitted on MI355X to calls over M = 33 .. 4096 against
 # weights of 1536 x 8960, 1536 x 1536, 4096 x 4096, 2560 x 2048, 512 x 512 (one weight, 1 to 16 K splits) and
 # 8960 x 1536, 4864 x 896, 11008 x 4096, 1024 x 512 (SiLU pairs), enough copies of them that they come from HBM:
 # a call takes 2 us and ceil(workgroups / (CUs x workgroups per CU)) rounds of (K / 64 steps + fixed), with K
@@ -91,12 +95,15 @@ CONV_NFAST = os.environ.get("HIPRT_CONV_NFAST", "1") == "1"   # conv tile order 
 # 29% high), and the plan it picks is 0.5% slower than the fastest on average, 11% at worst (SiLU at
 # 3000 x 1024 x 512). Launches inside a layer, with other kernels before them, take 5-20% longer.
 TILE_COST = {
-    "silu": {(64, 64, 8): (0.4, 1.5, 0.8), (128, 80, 10): (0.68, 3.1), (128, 144, 12): (1.02, 3.75),
+    "silu": {(64, 64, 8): (0.4, 1.5, 0.8, 1.5), (128, 80, 10): (0.68, 3.1), (128, 144, 12): (1.02, 3.75),
              (192, 144, 12): (1.39, 4.75), (256, 144, 12): (1.64, 5.5)},
-    "one": {(64, 64, 8): (0.2, 2.2, 0.39), (64, 96, 8): (0.32, 1.6), (128, 96, 8): (0.46, 1.7), (128, 128, 8): (0.535, 2.6),
+    "one": {(64, 64, 8): (0.2, 2.2, 0.39, 2.2), (64, 96, 8): (0.32, 1.6), (128, 96, 8): (0.46, 1.7), (128, 128, 8): (0.535, 2.6),
             (256, 128, 8): (0.82, 3.8), (256, 256, 8): (1.45, 7.0)},
-    "conv": {(64, 64, 8): (0.35, 2.1, 0.55), (64, 128, 8): (0.45, 2.8), (128, 128, 8): (0.66, 2.8)},   # tap gathers
-    "grp": {(64, 64, 8): (0.21, 2.1, 0.36), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.5, 2.6)},
+    "conv": {(64, 64, 8): (0.35, 2.1, 0.42, 5.5), (64, 128, 8): (0.45, 2.8), (128, 128, 8): (0.66, 2.8)},   # tap gathers
+    # the image's own rows (1 x 1): no addresses to make; 2048 -> 2048 on 16 x 16, with the conv before it: 29.4 us on
+    # 64 x 64 unsplit, 32.8 on 64 x 128 with 4 K splits, which the gathers' rates ask for
+    "conv1": {(64, 64, 8): (0.2, 2.2, 0.36, 2.2), (64, 128, 8): (0.36, 2.8), (128, 128, 8): (0.535, 2.6)},
+    "grp": {(64, 64, 8): (0.21, 2.1, 0.36, 2.1), (64, 128, 8): (0.33, 2.8), (128, 128, 8): (0.5, 2.6)},
 }
 # us, us per byte of partials, per split (o_proj 128 x 1536 x 1536: 9.3 us with 4 splits, 9.9 with 5),
 # and for a second round of 8 splits' loads
@@ -109,17 +116,19 @@ TILE_MAX_PART = 256 << 20   # bytes of fp32 partials one launch may use
 def tile_us(kind: str, tile: tuple, wgs: int, steps: int) -> float:
     """us that TILE_COST gives ``wgs`` workgroups of ``steps`` K steps each."""
     step, fixed, *shared = TILE_COST[kind][tile]
+    alone = steps * step + fixed
     if not shared:
-        return -(-wgs // TILE_CUS) * (steps * step + fixed)
+        return -(-wgs // TILE_CUS) * alone
+    both = steps * shared[0] + shared[1]
     full, rest = divmod(wgs, 2 * TILE_CUS)
-    last = 0.0 if not rest else steps * (shared[0] if rest > TILE_CUS else step) + fixed
-    return full * (steps * shared[0] + fixed) + last
+    return full * both + (both if rest > TILE_CUS else alone if rest else 0.0)
 
 
 def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follows: bool = False) -> tuple[int, int, int, int]:
     """(BM, BN, waves, K splits) of the tile.hip kernel that TILE_COST expects to be fastest for an
     M x N x K GEMM, K % 64 == 0. ``kind``: "silu" (two weights), "one", or "grp" (columns of several
-    weights: BN divides every group boundary in ``bounds``), "conv"; "one" and "conv" split K.
+    weights: BN divides every group boundary in ``bounds``), "conv" (gathered taps), "conv1" (1 x 1); all but
+    "silu" and "grp" split K.
     ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
     (k_gemm_reduce_*_resid_norm), so it costs little more than its bytes. The line between
     two tiles lies where the rounds of workgroups make the smaller one cheaper. SiLU at N = 8960,
@@ -133,7 +142,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
         if any(b % bn for b in bounds):
             continue
         tiles = -(-M // bm) * -(-N // bn)
-        for ks in range(1, TILE_MAX_SPLIT + 1 if kind in ("one", "conv") else 2):
+        for ks in range(1, TILE_MAX_SPLIT + 1 if kind in ("one", "conv", "conv1") else 2):
             steps = -(-(K // 64) // ks)
             if ks > 1 and (steps * 64 < GEMM_MIN_KCHUNK or -(-(K // 64) // steps) != ks
                            or ks * M * N * 4 > TILE_MAX_PART or tiles * ks > 2 * TILE_CUS):
@@ -1219,10 +1228,11 @@ class Lowering:
         flags = (1 if has_bias else 0) | (2 if bn is not None else 0) | (4 if rv is not None else 0) | (8 if relu else 0)
         if CONV_NFAST and xv.numel > Cout * K:   # input larger than the weights: N tiles fastest
             flags |= 16
-        tile = K > CONV_TILE_MIN_K and -(-M // 64) * -(-Cout // 64) >= CONV_TILE_MIN_WGS
+        tiles = -(-M // 64) * -(-Cout // 64)
+        tile = K > CONV_TILE_MIN_K and tiles >= CONV_TILE_MIN_WGS and (Cout > 64 or tiles <= CONV_TILE_NARROW_WGS)
         gn = 1
         if tile:
-            bm, bn_, waves, ksplit = tile_plan(M, Cout, K, "conv")
+            bm, bn_, waves, ksplit = tile_plan(M, Cout, K, "conv1" if plain else "conv")
             gn = -(-Cout // bn_) if flags & 16 else tile_group(M, Cout, bm, bn_, 1, ksplit)
         else:
             bm, bn_, ksplit = conv_gemm_tiling(M, Cout, K)
@@ -1230,7 +1240,7 @@ class Lowering:
         # takes the 2-stage variant, whose smaller LDS footprint lets more workgroups share a CU
         # (the 56 x 56 3 x 3 convs, K = 576: 28 -> 25.5 us)
         stages = "d2" if K <= CONV_D2_MAX_K or (bm, bn_) != (64, 64) else "d"
-        if plain and (bm, bn_) == (64, 64) and -(-M // 64) * -(-Cout // 64) * ksplit <= CONV_D_WGS:
+        if plain and (bm, bn_) == (64, 64) and tiles * ksplit <= CONV_D_WGS:
             stages = "d"   # a CU to itself: the loads in flight count, not the footprint
         if plain and K <= CONV_D1_MAX_K and (bm, bn_) == (64, 64) and ksplit == 1:
             stages = "d1"   # few K steps: one stage of LDS (16 KB), up to eight workgroups per CU

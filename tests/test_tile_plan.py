@@ -53,13 +53,30 @@ def test_rows_just_past_a_full_round(kind, N, K, rows, tile):
 
 
 def test_two_workgroups_per_cu_are_one_round():
-    """The third number of a TILE_COST entry: 257 to 512 workgroups are one round of shared CUs, and what is
+    """The second pair of a TILE_COST entry: 257 to 512 workgroups are one round of shared CUs, and what is
     left of a round goes at the rate of a CU to each."""
     from hip_compiler.subgraph_analyzer import TILE_COST, tile_us
 
     tile = (64, 64, 8)
-    step, fixed, shared = TILE_COST["one"][tile]
-    for wgs, us in ((1, step), (256, step), (257, shared), (512, shared)):
-        assert tile_us("one", tile, wgs, 10) == pytest.approx(10 * us + fixed)
-    assert tile_us("one", tile, 600, 10) == pytest.approx(10 * (shared + step) + 2 * fixed)
+    step, fixed, step2, fixed2 = TILE_COST["one"][tile]
+    alone, both = 10 * step + fixed, 10 * step2 + fixed2
+    for wgs, us in ((1, alone), (256, alone), (257, both), (512, both), (600, both + alone), (1024, 2 * both)):
+        assert tile_us("one", tile, wgs, 10) == pytest.approx(us)
     assert tile_us("one", (128, 128, 8), 257, 10) == pytest.approx(2 * tile_us("one", (128, 128, 8), 256, 10))
+
+
+@pytest.mark.parametrize("N,HW,C,Cout,k,kernel,ksplit", [
+    (4, 56, 128, 64, 3, "k_gemm_f16_convg_m64n64_w8_k64d", 1),        # 196 tiles of 64 x 64: within a round
+    (11, 56, 128, 64, 3, "k_gemm_f16_convg_m128n64_k64d2", 1),        # 539: no half-empty 128-column tiles
+    (64, 28, 256, 32, 3, "k_gemm_f16_convg_m128n64_k64d2", 1),
+    (16, 56, 128, 72, 3, "k_gemm_f16_convg_m128n128_w8_k64d", 1),
+    (16, 56, 1088, 64, 1, "k_gemm_f16_conv_m128n64_k64d2", 1),
+    (1, 16, 2048, 2048, 1, "k_gemm_f16_conv_m64n64_w8_k64d", 1),      # the gathers' rates split K four ways here
+])
+def test_long_k_convolutions_take_the_tiles_that_fit_their_channels(N, HW, C, Cout, k, kernel, ksplit):
+    from hip_compiler import compile_subgraph
+    from test_gpu_parity import _conv_chain_ir
+
+    prog = compile_subgraph(_conv_chain_ir(N, 64, HW, HW, C, Cout, k, 1, k // 2, False))
+    (step,) = [s for s in prog.steps if s.kind == "conv" and s.args.get("N") == Cout and s.module in ("gemm", "tile")]
+    assert (step.kernel, step.args["ksplit"]) == (kernel, ksplit)
