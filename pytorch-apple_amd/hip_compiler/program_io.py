@@ -77,6 +77,8 @@ def program_to_dict(prog: HIPProgram) -> dict:
 
 
 def program_from_dict(data: dict) -> HIPProgram:
+    from hip_runtime.kernels import builtin_kernels
+
     if data.get("format") != FORMAT or data.get("version") != VERSION:
         raise ValueError(f"not a {FORMAT} v{VERSION} file")
     body = data["program"]
@@ -84,6 +86,13 @@ def program_from_dict(data: dict) -> HIPProgram:
     if set(body) != names:
         raise ValueError(f"program fields differ: {sorted(set(body) ^ names)}")
     prog = HIPProgram(**{k: _dec(v) for k, v in body.items()})
+    # kernels come and go with the builds: a file may name one that the built modules no longer hold
+    generated = {ks.kernel_name for ks in prog.kernel_sources}
+    for step in prog.steps:
+        names = None if step.module in generated else builtin_kernels(step.module)
+        if names is not None and step.kernel not in names:
+            raise ValueError(f"module {step.module!r} holds no kernel {step.kernel!r}: the program was compiled for "
+                             "other kernels, compile it again")
     # k_mask_extent writes two ints per 32-query block; files written when it wrote one hold half the bytes
     for step in prog.steps:
         if step.kernel == "k_mask_extent":

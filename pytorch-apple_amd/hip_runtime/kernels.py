@@ -12,8 +12,10 @@ with ``hs_argsize`` from the shim.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import hashlib
 import os
+import re
 
 from hip_runtime import _shim
 
@@ -141,6 +143,21 @@ def kernel_cache_dir() -> str:
     d = os.environ.get("HIPRT_KCACHE", os.path.join(_shim.PKG, ".kcache"))
     os.makedirs(d, exist_ok=True)
     return d
+
+
+@functools.lru_cache(maxsize=None)
+def _kernel_names(path: str, mtime_ns: int) -> frozenset[str]:
+    with open(path, "rb") as f:
+        return frozenset(n.decode() for n in re.findall(rb"([A-Za-z_]\w*)\.kd\0", f.read()))
+
+
+def builtin_kernels(module: str) -> frozenset[str] | None:
+    """Names of the kernels in a built module (its kernel descriptors' symbols), None where it is not built."""
+    path = os.path.join(_shim.KERNEL_DIR, module + ".hsaco")
+    try:
+        return _kernel_names(path, os.stat(path).st_mtime_ns)
+    except FileNotFoundError:
+        return None
 
 
 class ModuleCache:

@@ -55,6 +55,44 @@ def test_hipbin_with_smaller_mask_extents_is_refused():
         program_from_dict(d)
 
 
+def test_hipbin_naming_a_kernel_that_is_gone_is_refused(tmp_path, monkeypatch):
+    """A file from a build whose kernels were since replaced, on load and not when its executor is made; the
+    cache compiles such an entry again. Modules that are not built here are not judged."""
+    from hip_runtime import _shim
+    from hip_runtime.kernels import builtin_kernels
+
+    ir = graphs()["prefill"]
+    prog = compile_subgraph(ir)
+    d = json.loads(json.dumps(program_to_dict(prog)))
+    modules = {s["module"] for s in d["program"]["steps"]} - {k["kernel_name"] for k in d["program"]["kernel_sources"]}
+    assert {"gemm", "attention"} <= modules
+    monkeypatch.setattr(_shim, "KERNEL_DIR", str(tmp_path))
+    assert builtin_kernels("gemm") is None and program_from_dict(d) == prog
+    for m in modules:
+        names = {s["kernel"] for s in d["program"]["steps"] if s["module"] == m}
+        (tmp_path / f"{m}.hsaco").write_bytes(b"\0".join(n.encode() + b".kd" for n in sorted(names)) + b"\0")
+    assert program_from_dict(d) == prog
+    step = next(s for s in d["program"]["steps"] if s["module"] == "gemm")
+    step["kernel"] += "_k64d"
+    with pytest.raises(ValueError, match="compile it again"):
+        program_from_dict(d)
+    save_program(prog, str(tmp_path / "p.hipbin"))
+    (tmp_path / "gemm.hsaco").write_bytes(b"k_other.kd\0")
+    with pytest.raises(ValueError, match="holds no kernel"):
+        load_program(str(tmp_path / "p.hipbin"))
+
+
+@pytest.mark.parametrize("name", ["decode", "prefill", "resnet"])
+def test_every_kernel_of_a_program_is_in_the_built_modules(name):
+    from hip_runtime.kernels import builtin_kernels
+
+    prog = compile_subgraph(graphs()[name])
+    generated = {k.kernel_name for k in prog.kernel_sources}
+    for step in prog.steps:
+        names = None if step.module in generated else builtin_kernels(step.module)
+        assert names is None or step.kernel in names, (step.module, step.kernel)
+
+
 def test_program_cache_hits_and_keys(tmp_path):
     ir = graphs()["decode"]
     a = compile_cached(ir, str(tmp_path))
