@@ -153,6 +153,13 @@ def lowering_settings(options: dict) -> dict:
         "conv_split_short_tiles": int(subgraph_analyzer.CONV_SPLIT_SHORT_TILES),
         "conv_tile_min_k": int(subgraph_analyzer.CONV_TILE_MIN_K),
         "conv_tile_min_wgs": int(subgraph_analyzer.CONV_TILE_MIN_WGS),
+        "conv_tile_narrow_wgs": int(subgraph_analyzer.CONV_TILE_NARROW_WGS),
+        # what picks the tiles and K splits of the wide-workgroup GEMMs
+        "tile_cost": {kind: {"x".join(map(str, t)): c for t, c in costs.items()}
+                      for kind, costs in subgraph_analyzer.TILE_COST.items()},
+        "tile_limits": [subgraph_analyzer.TILE_REDUCE, subgraph_analyzer.TILE_CUS, subgraph_analyzer.TILE_MAX_SPLIT,
+                        subgraph_analyzer.TILE_MAX_PART, subgraph_analyzer.GEMM_MIN_KCHUNK,
+                        subgraph_analyzer.GEMM_TARGET_WGS],
         "prefill_attn_wgs": int(patterns.PREFILL_ATTN_WGS),
         "conv_d1_max_k": subgraph_analyzer.CONV_D1_MAX_K,
         "fuse_reduce_norm": bool(patterns.FUSE_REDUCE_NORM),
@@ -161,6 +168,8 @@ def lowering_settings(options: dict) -> dict:
         "decode_kv_major_min_s": int(persistent.KV_MAJOR_MIN_S),
         "decode_slot_combine": bool(persistent.SLOT_COMBINE),
         "skinny_min_m": int(subgraph_analyzer.SKINNY_MIN_M),
+        "skinny_max_m": int(subgraph_analyzer.SKINNY_MAX_M),
+        "gemm_min_m": int(subgraph_analyzer.GEMM_MIN_M),
         "skinny_norm_max_k": int(subgraph_analyzer.SKINNY_NORM_MAX_K),
         "wide_max_m": int(subgraph_analyzer.WIDE_MAX_M),
         "wide_halves": bool(subgraph_analyzer.WIDE_HALVES),

@@ -160,3 +160,18 @@ def test_cache_key_covers_lowering_switches(monkeypatch):
     assert cache_key(ir, {}) == base
     monkeypatch.setattr(subgraph_analyzer, "CONV_NFAST", not subgraph_analyzer.CONV_NFAST)
     assert cache_key(ir, {}) != base
+
+
+@pytest.mark.parametrize("name,value", [
+    ("TILE_COST", {"silu": {(64, 64, 8): (1.0, 1.0)}}), ("TILE_REDUCE", (0.0, 0.0, 0.0, 0.0)), ("TILE_CUS", 128),
+    ("TILE_MAX_SPLIT", 1), ("TILE_MAX_PART", 0), ("GEMM_MIN_KCHUNK", 64), ("GEMM_TARGET_WGS", 128),
+    ("CONV_TILE_NARROW_WGS", 0), ("CONV_TILE_MIN_K", 64), ("CONV_TILE_MIN_WGS", 1), ("CONV_D_WGS", 0),
+    ("CONV_SPLIT_SHORT_TILES", 0), ("CONV_D1_MAX_K", 0), ("CONV_SMALL_TILE_MAX_K", 0), ("SKINNY_MAX_M", 8),
+    ("GEMM_MIN_M", 1)])
+def test_cache_key_covers_what_picks_the_kernels(name, value, monkeypatch):
+    from hip_compiler import subgraph_analyzer
+
+    ir = graphs()["prefill"]
+    base = cache_key(ir, {})
+    monkeypatch.setattr(subgraph_analyzer, name, value)
+    assert cache_key(ir, {}) != base
