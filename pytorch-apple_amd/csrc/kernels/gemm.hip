@@ -750,9 +750,6 @@ __device__ __forceinline__ void reduce_norm_body(const ReduceNormArgs& a) {
 extern "C" __global__ void __launch_bounds__(256) k_gemm_reduce_bf16_resid_norm(const ReduceNormArgs a) {
   reduce_norm_body<HS_BF16>(a);
 }
-extern "C" __global__ void __launch_bounds__(256) k_gemm_reduce_f16_resid_norm(const ReduceNormArgs a) {
-  reduce_norm_body<HS_F16>(a);
-}
 
 // up to 2 waves per SIMD: the 64 accumulator registers plus staging and fragments need
 // more than the default register budget, which would otherwise spill the staging to scratch

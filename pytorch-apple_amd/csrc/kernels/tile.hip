@@ -36,7 +36,7 @@
 //   RESID out = round(r + round(acc + b))
 //   SILU  out = round(round(silu(round(acc_g + b_g))) * round(acc_u + b_u))   (NW = 2)
 //   CONV  round(acc + b), batch norm, residual and ReLU as gemm.hip's conv epilogue
-// ksplit > 1: grid.z workgroups take kchunk of K each and store fp32 partials [z, NW, M, N]; a
+// ksplit > 1 (NW = 1): grid.z workgroups take kchunk of K each and store fp32 partials [z, M, N]; a
 // k_gemm_reduce_* kernel (gemm.hip) sums them in order and applies the epilogue.
 // CV: x rows are gathered from an NHWC image, one tap and 64 channels per stage (K = (kh, kw, ci),
 // cCin % 64 == 0), taps outside it from a.zero. ResNet-50's 3 x 3 convs at batch 32 with 128 / 256 / 512
@@ -222,26 +222,24 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
 
   // this lane's part of a 16 x 16 tile: row fr, columns cn .. cn + 3
   const int cn = 4 * fc;
-  if (a.ksplit > 1) {
+  if (NW == 1 && a.ksplit > 1) {
 #pragma unroll
-    for (int u = 0; u < NW; ++u)
+    for (int i = 0; i < TI; ++i) {
+      const int m = m_base + wr * WM + i * 16 + fr;
+      if (m >= M) continue;
+      float* p = a.part + ((long long)kz * a.M + m) * N;
 #pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        const int m = m_base + wr * WM + i * 16 + fr;
-        if (m >= M) continue;
-        float* p = a.part + (((long long)kz * NW + u) * a.M + m) * N;
+      for (int j = 0; j < TJ; ++j) {
+        const int n = n_base + wc * WN + j * 16 + cn;
+        if ((N & 3) == 0) {
+          if (n < N) *(tg_f32x4*)(p + n) = acc[0][j][i];
+        } else {
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-          const int n = n_base + wc * WN + j * 16 + cn;
-          if ((N & 3) == 0) {
-            if (n < N) *(tg_f32x4*)(p + n) = acc[u][j][i];
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < N) p[n + e] = acc[u][j][i][e];
-          }
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) p[n + e] = acc[0][j][i][e];
         }
       }
+    }
     return;
   }
   // epilogue: the rounded tile through LDS (round(acc + bias) is the first rounding point, so a

@@ -25,7 +25,7 @@ from hip_compiler.program import DTYPE_CODE, LaunchStep
 from npu_compiler.ir_reader import OpNode
 
 # a split-K reduce with the residual epilogue and the RMSNorm reading its result run as one
-# kernel (k_gemm_reduce_*_resid_norm); off = two launches with the same results
+# kernel (k_gemm_reduce_bf16_resid_norm); off = two launches with the same results
 FUSE_REDUCE_NORM = True
 
 # workgroups of prefill attention up to which a workgroup takes fewer heads (one per CU; 512 tokens of
@@ -144,7 +144,7 @@ def rmsnorm(low) -> None:
                     and prev.args["ldo"] == cols and prev.args["out"] == low.ref(xv)):
                 pa = prev.args
                 low.steps[-1] = LaunchStep(
-                    kind="gemm", kernel=f"k_gemm_reduce_{'bf16' if xv.dtype == 'bfloat16' else 'f16'}_resid_norm",
+                    kind="gemm", kernel="k_gemm_reduce_bf16_resid_norm",
                     module="gemm", arg_struct="ReduceNormArgs",
                     args=dict(part=pa["part"], bias=pa["bias"] if pa["flags"] & 1 else None, resid=pa["resid"],
                               out=pa["out"], norm_w=low.ref(wv), norm_out=low.ref(o), M=rows, ldr=pa["ldr"],

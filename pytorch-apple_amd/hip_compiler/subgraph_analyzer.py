@@ -130,7 +130,7 @@ def tile_plan(M: int, N: int, K: int, kind: str, bounds: tuple = (), norm_follow
     weights: BN divides every group boundary in ``bounds``), "conv" (gathered taps), "conv1" (1 x 1); all but
     "silu" and "grp" split K.
     ``norm_follows``: a reduce would also be the RMSNorm launch that follows anyway
-    (k_gemm_reduce_*_resid_norm), so it costs little more than its bytes. The line between
+    (k_gemm_reduce_bf16_resid_norm), so it costs little more than its bytes. The line between
     two tiles lies where the rounds of workgroups make the smaller one cheaper. SiLU at N = 8960,
     K = 1536: 128 x 80 tiles up to M = 256 (224 workgroups, 24 us; 128 x 144 33), 128 x 144 up to 512 (252, 34 us;
     192 x 144 44), 192 x 144 up to 768 (252, 45 us; 128 x 144 48, 256 x 144 51) and again at 1025 .. 1536
@@ -538,7 +538,7 @@ class Lowering:
                            epi="bias", nodes=[node.name])
             return
         self.emit_linear(x_t.name, w_t.name, b_t.name if b_t else None, out.name, tuple(out.shape), out.dtype,
-                         resid=None, node_names=[node.name])
+                         [node.name])
 
     # ------------------------------------------------------------------ fused decode GEMV
 
@@ -843,7 +843,7 @@ class Lowering:
         self.views[out_name] = o
 
     def emit_linear(self, x_name: str, w_name: str, b_name: str | None, out_name: str, out_shape, out_dtype: str,
-                    resid: str | None, node_names: list[str]) -> None:
+                    node_names: list[str]) -> None:
         x = self.contiguous(x_name)
         w = self.contiguous(w_name)
         K = x.shape[-1]
@@ -855,25 +855,21 @@ class Lowering:
             ok = ok and self.view(b_name).dtype == out_dtype
         if not ok:
             self.emit_linear_generic(x, w, b_name, out_name, out_shape, out_dtype, node_names)
-            if resid is not None:
-                raise NotImplementedError("residual epilogue on the generic path")
             return
         if M >= GEMM_MIN_M and K % 32 == 0 or skinny_rows(M, K, out_dtype):
-            self.emit_gemm(x_name, w_name, b_name, out_name, out_shape, out_dtype,
-                           epi="resid" if resid is not None else "bias", nodes=node_names, resid=resid)
+            self.emit_gemm(x_name, w_name, b_name, out_name, out_shape, out_dtype, epi="bias", nodes=node_names)
             return
         o = self.new_storage(out_name, out_shape, out_dtype)
         bias = self.contiguous(b_name) if b_name is not None else None
-        r = self.contiguous(resid) if resid is not None else None
         mb, rpw = (1, 4) if M <= 1 else (4, 2)
         kname = f"k_linear_{'bf16' if out_dtype == 'bfloat16' else 'f16'}_m{mb}"
         self.emit(LaunchStep(
             kind="gemm", kernel=kname, module="linear", arg_struct="LinearArgs",
             args=dict(x=self.ref(x), w=self.ref(w), bias=self.ref(bias) if bias else None, out=self.ref(o),
-                      resid=self.ref(r) if r else None, M=M, ldx=K, ldo=N, ldr=N, N=N, K=K,
-                      dtype=DTYPE_CODE[out_dtype], has_bias=int(bias is not None), has_resid=int(r is not None)),
+                      resid=None, M=M, ldx=K, ldo=N, ldr=N, N=N, K=K,
+                      dtype=DTYPE_CODE[out_dtype], has_bias=int(bias is not None), has_resid=0),
             grid=((N + 4 * rpw - 1) // (4 * rpw), (M + mb - 1) // mb, 1),
-            inputs=[x_name, w_name] + ([b_name] if b_name else []) + ([resid] if resid else []),
+            inputs=[x_name, w_name] + ([b_name] if b_name else []),
             outputs=[out_name], params={"M": M, "N": N, "K": K, "has_bias": bias is not None,
                                         "transpose_b": True, "nodes": node_names}))
         self.views[out_name] = o
@@ -1012,7 +1008,7 @@ class Lowering:
             # mat2 is W^T of a contiguous W[N, K]
             wname = m2 + ".T"
             self.views[wname] = V.transpose(w2, 0, 1)
-            self.emit_linear(m1, wname, bias, out.name, tuple(out.shape), out.dtype, None, [node.name])
+            self.emit_linear(m1, wname, bias, out.name, tuple(out.shape), out.dtype, [node.name])
             return
         a, b = self.view(m1), self.view(m2)
         o = self.new_storage(out.name + ".mm", out.shape, out.dtype)
