@@ -605,6 +605,22 @@ struct AttnOutArgs {          // second attention pass: global softmax and p.V p
 #define HS_HD
 #endif
 
+// tile.hip's order of tiles. Workgroup lin of a gx x gy x gz grid (column tiles, row tiles, K splits) runs on XCD
+// lin % 8, so lin is remapped to give each XCD a contiguous range of tiles, ordered in groups of gn column
+// tiles, row tiles next, columns within the group fastest: the range is then a block of about gn columns,
+// whose weights and activations the XCD's L2 fetches once
+struct TilePos {
+  unsigned col, row, kz;
+};
+HS_HD inline TilePos tile_order(unsigned lin, unsigned gx, unsigned gy, unsigned gz, unsigned gn) {
+  const unsigned total = gx * gy * gz, per = (total + 7) / 8, xcd = lin % 8, loc = lin / 8;
+  const unsigned tall = total % 8 == 0 ? 8 : total % 8;   // XCDs that get `per` tiles; the rest get per - 1
+  const unsigned tile = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+  const unsigned kz = tile / (gx * gy), t2 = tile - kz * gx * gy;
+  const unsigned first = t2 / (gn * gy) * gn, width = gx - first < gn ? gx - first : gn, t3 = t2 - first * gy;
+  return TilePos{first + t3 % width, t3 / width, kz};
+}
+
 // sin and cos of an fp32 angle (|x| < 2^30), branch-free and table-free so that no load or
 // wait enters the caller's critical path: Cody-Waite reduction by pi/2 in double (k*pi/2 with
 // a two-part pi/2), Taylor polynomials in double on |r| <= pi/4 (truncation error < 1e-17),
@@ -989,8 +1005,8 @@ __device__ __forceinline__ float gm_hi(uint32_t w) {
 // an IEEE division take about 25, and an epilogue is 10 us of a 1000 x 8960 output's 53): both
 // sides of the fraction scaled by 1/4 so that the reciprocal stays a normal number down to v = -88.7
 // (where expf overflows), one remainder step on the quotient (skipped where the remainder is zero or
-// NaN: v = -0, and the infinities). Over all 2^16 inputs its rounding to 16 bits differs from the
-// correctly rounded result as often as the library form's does: 17 times in bfloat16, once in float16.
+// NaN: v = -0, and the infinities). Over all bfloat16 inputs its rounding differs from the correctly
+// rounded result 17 times, as often as the library form's does.
 __device__ __forceinline__ float gm_silu(float v) {
   const float d = 0.25f + __builtin_amdgcn_exp2f(__builtin_fmaf(v, -1.44269504088896340736f, -2.f));
   const float v4 = 0.25f * v, r = __builtin_amdgcn_rcpf(d), q = v4 * r, rem = __builtin_fmaf(-q, d, v4);

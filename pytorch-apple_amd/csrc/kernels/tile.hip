@@ -79,18 +79,10 @@ __device__ __forceinline__ void tile_body(const GemmArgs& a) {
   __shared__ __attribute__((aligned(16))) float Fb[(EPI == GE_CONV ? 3 : NW) * BN];   // bias per weight; conv: bias, al, be
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave / WC, wc = wave % WC;
-  // XCD-aware tile order: workgroup L runs on XCD L % 8, so L is remapped to give each XCD a contiguous
-  // range of tiles, ordered in groups of gn column tiles, row tiles next, columns within the group
-  // fastest: the range is then a block of about gn columns, whose weights and activations the XCD's
-  // L2 fetches once
-  const unsigned gx = gridDim.x, gy = gridDim.y, total = gx * gy * gridDim.z;
-  const unsigned lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-  const unsigned per = (total + 7) / 8, xcd = lin % 8, loc = lin / 8;
-  const unsigned tall = total % 8 == 0 ? 8 : total % 8;   // XCDs that get `per` tiles; the rest get per - 1
-  const unsigned tile = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
-  const unsigned kz = tile / (gx * gy), t2 = tile - kz * gx * gy, gn = (unsigned)max(a.gn, 1);
-  const unsigned grp0 = t2 / (gn * gy) * gn, gw = min(gn, gx - grp0), t3 = t2 - grp0 * gy;
-  const int m_base = (int)(t3 / gw) * BM, n_base = (int)(grp0 + t3 % gw) * BN;
+  const TilePos at = tile_order(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y,
+                                gridDim.z, (unsigned)max(a.gn, 1));
+  const unsigned kz = at.kz;
+  const int m_base = (int)at.row * BM, n_base = (int)at.col * BN;
   const int M = (int)a.M, N = a.N;
   const int kbeg = (int)kz * a.kchunk, nsteps = min(a.kchunk, a.K - kbeg) / 64;
   int g_lo = 0, g_hi = N;   // GRP: the columns of this tile's group

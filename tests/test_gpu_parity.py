@@ -764,6 +764,64 @@ def test_prefill_chunk_ragged_vs_cpu_and_oracle(backend):
         assert np.array_equal(np.asarray(got[name])[:, :, keep], np.asarray(x[f"past_{kind}_0"])[:, :, keep])
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(6, 1), (5, 1), (3, 3)])
+def test_prefill_rope_waves_that_mix_heads(backend, heads, kv_heads):
+    """k_rope_cache takes four heads of a token per wave: head counts whose groups hold the last q heads with k
+    and v (6 + 1 + 1), end in a part of a group (5 + 1 + 1: seven) and do both (3 + 3 + 3: nine), at cache
+    positions past the first, against the CPU fallback."""
+    from irgen.qwen import QwenConfig, build_decode_ir
+    from irgen.workloads import make_weights, prefill_inputs
+
+    cfg = QwenConfig(hidden=heads * 128, intermediate=512, layers=1, heads=heads, kv_heads=kv_heads, vocab=512)
+    T, S, P0 = 35, 64, 20
+    ir = build_decode_ir(S, cfg, argmax=True, tokens=T)
+    w = host(make_weights(ir, cfg))
+    x = prefill_inputs(T, S, cfg)
+    at = torch.arange(P0, P0 + T, dtype=torch.int64)
+    m = torch.zeros(T, S).masked_fill_(torch.arange(S)[None, :] > at[:, None], float("-inf"))
+    x.update(position_ids=at.reshape(1, T), cache_position=at, attention_mask=m.bfloat16().reshape(1, 1, T, S))
+    x = host(x)
+    print(f"[case] prefill RoPE {heads} q heads, {kv_heads} kv heads", flush=True)
+    got, ex = run_hip(ir, x, w, backend)
+    assert "k_rope_cache" in [st.kernel for p in ex.npu_programs.values() for st in p.steps]
+    ref = run_cpu(ir, x, w)
+    for o in ir["graph_outputs"][:-1]:
+        close(got[o["name"]], ref[o["name"]])
+
+
+@pytest.mark.parametrize("N,C,H,W,dtype", [
+    (3, 72, 9, 7, "float16"),     # 63 pixels: a second round of 56; nine chunks of 8 channels, a wave takes eight
+    (2, 72, 8, 8, "bfloat16"),    # 64 pixels
+    (1, 64, 7, 8, "float16"),     # exactly one round
+    (5, 128, 1, 1, "float16"),    # one pixel
+    (2, 200, 13, 11, "float16"),  # 143 pixels: three rounds
+])
+def test_global_pool_channels_last(backend, N, C, H, W, dtype):
+    """k_mean_nhwc over a conv's channels-last output, against the float64 mean of that output: one rounding
+    (u = 2^-11, 2^-8 for bfloat16) and H W fp32 additions."""
+    from irgen.builder import IRBuilder
+
+    b = IRBuilder("pool")
+    y = b.input("x", [N, 64, H, W], dtype)
+    attrs = {"stride": [1, 1], "padding": [0, 0], "dilation": [1, 1], "groups": 1}
+    for i, (co, ci) in enumerate(((64, 64), (C, 64))):
+        y = b.op("aten.conv2d.default", [y, b.weight(f"w{i}", [co, ci, 1, 1], dtype)], attrs)
+    p = b.op("aten.adaptive_avg_pool2d.default", [y], {"output_size": [1, 1]})
+    b.output(y, p)
+    ir = b.to_dict()
+    g, td = torch.Generator().manual_seed(C + H), getattr(torch, dtype)
+    w = {f"w{i}": (torch.randn(co, 64, 1, 1, generator=g) / 8).to(td) for i, co in enumerate((64, C))}
+    print(f"[case] global pool {N}x{C}x{H}x{W} {dtype}", flush=True)
+    got, ex = run_hip(ir, host({"x": torch.randn(N, 64, H, W, generator=g).to(td)}), host(w), backend)
+    assert "k_mean_nhwc_" + ("f16" if dtype == "float16" else "bf16") in \
+        [st.kernel for pr in ex.npu_programs.values() for st in pr.steps]
+    yv, pv = (f32(got[o["name"]]).astype(np.float64) for o in ir["graph_outputs"])
+    ref = yv.mean((2, 3), keepdims=True)
+    u = 2.0 ** -11 if dtype == "float16" else 2.0 ** -8
+    tol = u * np.abs(ref) + H * W * 2.0 ** -24 * np.abs(yv).mean((2, 3), keepdims=True) + 2.0 ** -24
+    assert (np.abs(pv - ref) <= tol).all()
+
+
 @pytest.mark.parametrize("transposed_b", [False, True])
 def test_batched_matmul_on_mfma(backend, transposed_b):
     """matmul over [2, 3] batches (attention-shaped) on the MFMA GEMM, b given as [K, N] or as the

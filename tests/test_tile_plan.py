@@ -1,23 +1,41 @@
 """The plan of the wide-workgroup GEMMs (hip_compiler tile_plan / tile_group) and their tile order, on the CPU."""
 
+import ctypes
+import os
+import shutil
+import subprocess
+
 import pytest
 
+HERE = os.path.dirname(os.path.abspath(__file__))
 
-def test_tile_order_covers_every_tile_once():
-    """The grouped tile order (tile.hip) over grids that do and do not divide by 8 or by the group:
-    every (row tile, column tile, split) exactly once."""
+
+@pytest.fixture(scope="module")
+def order(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    so = str(tmp_path_factory.mktemp("order") / "liborder.so")
+    subprocess.run(["g++", "-O2", "-shared", "-fPIC", "-I", os.path.join(HERE, "..", "pytorch-apple_amd", "csrc", "kernels"),
+                    os.path.join(HERE, "tile_host.cpp"), "-o", so], check=True)
+    lib = ctypes.CDLL(so)
+
+    def f(gx, gy, gz, gn):
+        out = (ctypes.c_uint * (3 * gx * gy * gz))()
+        lib.order(gx, gy, gz, gn, out)
+        return [tuple(out[i:i + 3]) for i in range(0, len(out), 3)]
+
+    return f
+
+
+def test_tile_order_covers_every_tile_once(order):
+    """The grouped tile order (tile.hip's own, built for the host) over grids that do and do not divide by 8 or by the
+    group: every (row tile, column tile, split) exactly once, and each XCD's share one stretch of the order."""
     for gx, gy, gz, gn in ((11, 16, 1, 5), (63, 8, 1, 1), (16, 16, 1, 7), (1, 1, 1, 1), (13, 3, 5, 4), (7, 9, 2, 7)):
-        total, seen = gx * gy * gz, set()
-        per, tall = -(-total // 8), 8 if total % 8 == 0 else total % 8
-        for lin in range(total):
-            xcd, loc = lin % 8, lin // 8
-            t = xcd * per + loc if xcd < tall else tall * per + (xcd - tall) * (per - 1) + loc
-            kz, t2 = divmod(t, gx * gy)
-            g0 = t2 // (gn * gy) * gn
-            gw = min(gn, gx - g0)
-            t3 = t2 - g0 * gy
-            seen.add((t3 // gw, g0 + t3 % gw, kz))
-        assert seen == {(m, n, z) for m in range(gy) for n in range(gx) for z in range(gz)}
+        tiles = order(gx, gy, gz, gn)
+        assert sorted(tiles) == [(m, n, z) for m in range(gy) for n in range(gx) for z in range(gz)]
+        in_order = [(m, n, z) for z in range(gz) for g in range(0, gx, gn) for m in range(gy)
+                    for n in range(g, min(g + gn, gx))]
+        assert [t for xcd in range(8) for t in tiles[xcd::8]] == in_order
 
 
 @pytest.mark.parametrize("kind,bounds", [("one", ()), ("silu", ()), ("grp", (1536, 1792)), ("grp", (512, 576))])
