@@ -7,7 +7,7 @@ concrete arena pointers, and record where external buffers (graph inputs and
 weights) must be patched in. ``run()`` resolves the external pointers; when they
 match the set packed last, the list is launched as it is (one host call per step,
 instead of the reference's one Python dispatch per IR step), launch by launch or, for
-long lists, as the HIP graph captured for that set; a new set re-packs the affected
+long lists and lists of short launches (``wants_graph``), as the HIP graph captured for that set; a new set re-packs the affected
 kernargs and, with graphs, captures one more. Up to
 ``MAX_GRAPHS`` graphs are kept, least recently used first out, so a loop whose
 first step reads one buffer and whose later steps read another (a decode loop
@@ -35,13 +35,19 @@ from hip_runtime.kernels import STRUCTS, ModuleCache
 
 _MODULES: dict[int, ModuleCache] = {}
 MAX_GRAPHS = 8
-# launch lists shorter than this are launched one by one (hs_replay), longer ones as one captured
-# graph. One call after the other, direct against graph: 2 launches (the MLP block of one token) 16.9
-# against 22.1 us, 3-4 (128 / 1000 rows) 44.9 / 96 against 46.0 / 104, 22 (two prefill layers of 2000
-# tokens) 732 against 769; 38 and 62 (prefill with the full head) 465 / 1056 against 471 / 1061, 80
-# (ResNet-50 at batch 1) 493 against 487. A call that is waited for: 2 launches 30 against 44 us,
-# 62 and 80 1086 / 526 against 1076 / 516, where the host's 1.5 us per launch begins to show.
+# Launch lists at least this long are launched as one captured graph, shorter ones launch by launch (hs_replay)
+# unless their launches are short. A graph costs about 5 us per call back to back and 8-16 us for a call that is
+# waited for (MLP block of one token, 2 launches: 16 / 21 and 29 / 40 us direct / graph); from 38 launches on that is
+# 1% or less either way (prefill of 128 tokens, 38 launches 445 / 452 and 462 / 467, 62 launches 673 / 679 and 692 / 696).
 GRAPH_MIN_STEPS = 33
+# Up to DIRECT_MAX_STEPS launches direct is faster whatever they take. From the eighth on the host stalls for about 15 us
+# in a list that starts on an idle device (and again later in long ones), which shows where the launches before
+# do not cover it: waited for, 12 / 32 launches of 3.3 us each take 59 / 154 us direct and 54 / 114 as a graph, 24 of
+# 4.3 us 129 and 118, a decode list of 28 (median below 4 us) 246 and 240; 22 of a 128-token prefill 306 and 314.
+# DIRECT_MIN_US lies between what launch_us makes of the lists that lost (2.7 - 4.8) and of those that gained or were
+# within 3% (5.0 on).
+DIRECT_MAX_STEPS = 7
+DIRECT_MIN_US = 4.9
 MAX_TABLES = 8   # pointer tables kept per executor without graphs (with graphs: all)
 
 
@@ -74,6 +80,22 @@ def resident_workgroups(device_index: int, module: str, kernel: str, threads: in
     return cus.value * per.value
 
 
+def launch_us(step, storages: dict) -> float:
+    """About what one launch takes: 2.5 us, the bytes of the storages it names at 5 TB/s, and 4 us of staging
+    and epilogue on matrix cores."""
+    named = {r.storage for r in _refs(step.args)}
+    mfma = step.params.get("mfma") or (step.kind == "attention" and step.params.get("T", 1) > 1)
+    return 2.5 + sum(storages[n].nbytes for n in named) * 0.2e-6 + (4.0 if mfma else 0.0)
+
+
+def wants_graph(program: HIPProgram) -> bool:
+    """Whether a launch list runs as a captured graph rather than launch by launch."""
+    n = len(program.steps)
+    if n >= GRAPH_MIN_STEPS or n <= DIRECT_MAX_STEPS:
+        return n >= GRAPH_MIN_STEPS
+    return sorted(launch_us(s, program.storages) for s in program.steps)[n // 2] < DIRECT_MIN_US
+
+
 class _HostFlags:
     """Host-visible 32-bit words that kernels set on failure (one per executor that needs one),
     carved out of pinned, coherent, device-mapped pages that are never freed."""
@@ -101,10 +123,11 @@ class HIPExecutor:
     def __init__(self, program: HIPProgram, backend=None, use_graph: bool | None = None):
         self.program = program
         self.device = backend.device if backend is not None else torch.device("cuda", torch.cuda.current_device())
+        self._graph_on_second = False
         if use_graph is None:
-            # a graph saves host time per launch and costs about 15 us before its first kernel: it pays
-            # for long lists only (GRAPH_MIN_STEPS)
-            use_graph = os.environ.get("HIPRT_NO_GRAPH", "0") != "1" and len(program.steps) >= GRAPH_MIN_STEPS
+            use_graph = os.environ.get("HIPRT_NO_GRAPH", "0") != "1" and wants_graph(program)
+            # a short list is captured when its pointers come a second time: a capture costs more than a launch of it
+            self._graph_on_second = use_graph and len(program.steps) < GRAPH_MIN_STEPS
         self.use_graph = use_graph
         mods = module_cache(self.device.index or 0)
         gen = {ks.kernel_name: ks.source_code for ks in program.kernel_sources}
@@ -163,6 +186,7 @@ class HIPExecutor:
         self._last_in_key: tuple = ()
         self._in_cache: OrderedDict[tuple, tuple] = OrderedDict()
         self._graphs: OrderedDict[tuple, int] = OrderedDict()   # (pointer set, advance) -> captured graph
+        self._seen: OrderedDict[tuple, None] = OrderedDict()    # the last sets launched directly (_graph_on_second)
         self._adv_ptr = 0                         # flag word of a decode advance folded into the launch
         self._adv_bufs: tuple = ()                # its (mask, position, cache position, mask bytes)
         self._adv_checked: tuple | None = None    # the (pointer set, advance) last checked
@@ -356,8 +380,12 @@ class HIPExecutor:
             if self._adv_ptr and self._adv_checked != (key, self._adv_bufs):   # once per pointer set
                 self._check_advance(key, self._adv_bufs)
                 self._adv_checked = (key, self._adv_bufs)
-            if not self.use_graph:
+            if not self.use_graph or (self._graph_on_second and gkey not in self._seen):
                 _shim.check(lib.hs_replay(self._recs, self._n, stream), "replay")
+                if self.use_graph:
+                    self._seen[gkey] = None
+                    while len(self._seen) > MAX_GRAPHS:
+                        self._seen.popitem(last=False)
                 return
             if self._capture_stream is None:
                 cs = C.c_void_p()

@@ -439,3 +439,21 @@ def test_persistent_step_rejects_caches_past_its_chunk_word():
 
     prog = compile_subgraph(build_decode_ir(65536 + 128, QwenConfig(layers=1), argmax=True))
     assert len(prog.steps) > 1
+
+
+def test_launch_lists_that_become_graphs():
+    """Up to seven launches and lists of long ones go launch by launch, lists of short ones and long lists as a graph."""
+    from hip_runtime.hip_executor import launch_us, wants_graph
+    from irgen.qwen import QwenConfig, build_decode_ir, build_mlp_ir
+
+    mini = QwenConfig(hidden=512, intermediate=1024, layers=2, heads=4, kv_heads=2, head_dim=128, vocab=4096)
+    two = QwenConfig(layers=2, vocab=4096)
+    for ir, n, graph in ((build_mlp_ir(1), (1, 7), False), (build_mlp_ir(1000), (1, 7), False),
+                         (build_decode_ir(256, mini, argmax=True), (8, 32), True),
+                         (build_decode_ir(512, two, argmax=True), (8, 32), True),
+                         (build_decode_ir(32, two, argmax=True, tokens=16), (8, 32), False),
+                         (build_decode_ir(2048, two, argmax=True, tokens=2000), (8, 32), False),
+                         (build_decode_ir(128, QwenConfig(layers=8, vocab=4096), argmax=True, tokens=128), (33, 99), True)):
+        prog = compile_subgraph(ir, persistent=False)
+        assert n[0] <= len(prog.steps) <= n[1]
+        assert wants_graph(prog) == graph, [launch_us(s, prog.storages) for s in prog.steps]

@@ -39,3 +39,33 @@ def test_direct_and_graph_launches_agree_when_buffers_change(backend):
         assert not torch.equal(out[0], out[1]) and not torch.equal(out[0], out[3])
         runs[graph] = out
     assert all(torch.equal(a, b) for a, b in zip(runs[False], runs[True]))
+
+
+def test_short_launches_become_a_graph_on_their_second_call(backend):
+    """A list of 13 short launches (a two-layer decode without the one-launch step): a pointer set's first call
+    is launched directly, its second captured and its third the same graph, with equal results; another set
+    starts directly again."""
+    from hip_compiler import compile_subgraph, is_hip_op_supported
+    from irgen.qwen import QwenConfig, build_decode_ir
+    from irgen.workloads import decode_inputs, make_weights
+    from npu_compiler import partition
+    from npu_runtime import DAGExecutor
+
+    cfg = QwenConfig(hidden=512, intermediate=1024, layers=2, heads=4, kv_heads=2, head_dim=128, vocab=4096)
+    ir = build_decode_ir(256, cfg, argmax=True)
+    ex = DAGExecutor(partition(ir, is_hip_op_supported), backend,
+                     compile_fn=lambda sub: compile_subgraph(sub, persistent=False))
+    ex.load_weights(make_weights(ir, cfg, device="cuda"))
+    (hexec,) = ex.npu_executors.values()
+    assert hexec.use_graph
+    sets = [{k: backend.allocate_buffer(v.cuda()) for k, v in decode_inputs(256, 100, cfg, seed=s).items()} for s in (1, 2)]
+    names, out, graphs = [o["name"] for o in ir["graph_outputs"]], [], []
+    for i in (0, 0, 0, 1, 0, 1):
+        print(f"[case] input set {i}", flush=True)
+        y = ex.execute(sets[i])
+        out.append([y[n].to_torch().clone() for n in names])
+        graphs.append(len(hexec._graphs))
+    assert graphs == [0, 1, 1, 1, 1, 2]
+    for i, j in ((0, 1), (0, 2), (0, 4), (3, 5)):
+        assert all(torch.equal(a, b) for a, b in zip(out[i], out[j]))
+    assert not torch.equal(out[0][0], out[3][0])
