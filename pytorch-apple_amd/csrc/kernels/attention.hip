@@ -526,6 +526,7 @@ __device__ __forceinline__ void prefill_attn_body(const PrefillAttnArgs& a) {
   // every bank; V's in slot c ^ (4 (r & 3) + 2 ((r >> 2) & 1)): so do the transposing reads of 4 rows
   constexpr int NI = (16 + HW - 1) / HW;
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void*)&lds[0] + (unsigned)(sp * PA_TILE);
+  // (32-bit row offsets: the host takes S up to 65,536, 16 MB of a KV head)
   auto issue = [&](int it, int lim) {   // past block lim - 1: read again, not used
     const int p0 = min(PA_KS * it + sp, lim - 1) * PA_BP;
     const unsigned dst = lds0 + (unsigned)((it & 1) * PA_KS * PA_TILE);

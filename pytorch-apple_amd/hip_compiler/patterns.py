@@ -291,7 +291,7 @@ def decode_attention(low) -> None:
             else tr.inputs[0]
         kvh = k_spec.shape[1]
         S = k_spec.shape[2]
-        if H % kvh or H // kvh > 8 or k_spec.shape[3] != D or S > 64 * 1024:
+        if H % kvh or H // kvh > 8 or k_spec.shape[3] != D or S > 64 * 1024:   # (k_attn_prefill: 32-bit offsets)
             continue
         add_dtype = add_n.outputs[0].dtype if mask_name is not None else dt
         if mask_name is not None and T > 1:
