@@ -370,7 +370,10 @@ class HIPExecutor:
             return
         lib = _shim.lib()
         gkey = (key, self._adv_ptr)
-        graph = self._graphs.get(gkey) if self.use_graph else None
+        # a caller that captures this stream gets the launches themselves: they may come again at any time, and a graph
+        # launched or made inside a capture would not be part of it
+        use_graph = self.use_graph and not torch.cuda.is_current_stream_capturing()
+        graph = self._graphs.get(gkey) if use_graph else None
         if graph is not None:
             self._graphs.move_to_end(gkey)
         else:
@@ -380,9 +383,9 @@ class HIPExecutor:
             if self._adv_ptr and self._adv_checked != (key, self._adv_bufs):   # once per pointer set
                 self._check_advance(key, self._adv_bufs)
                 self._adv_checked = (key, self._adv_bufs)
-            if not self.use_graph or (self._graph_on_second and gkey not in self._seen):
+            if not use_graph or (self._graph_on_second and gkey not in self._seen):
                 _shim.check(lib.hs_replay(self._recs, self._n, stream), "replay")
-                if self.use_graph:
+                if use_graph:
                     self._seen[gkey] = None
                     while len(self._seen) > MAX_GRAPHS:
                         self._seen.popitem(last=False)

@@ -69,3 +69,46 @@ def test_short_launches_become_a_graph_on_their_second_call(backend):
     for i, j in ((0, 1), (0, 2), (0, 4), (3, 5)):
         assert all(torch.equal(a, b) for a, b in zip(out[i], out[j]))
     assert not torch.equal(out[0][0], out[3][0])
+
+
+@pytest.mark.parametrize("layers", [2, 7])
+def test_calls_inside_a_callers_capture(backend, layers):
+    """A list that runs as a graph by default (13 short launches, and more than 32), captured by its caller after
+    calls that made the executor's own graph: every replay, with eager work and a synchronisation between, equals
+    the eager result for the inputs the buffers hold then."""
+    from hip_compiler import compile_subgraph, is_hip_op_supported
+    from irgen.qwen import QwenConfig, build_decode_ir
+    from irgen.workloads import decode_inputs, make_weights
+    from npu_compiler import partition
+    from npu_runtime import DAGExecutor
+
+    cfg = QwenConfig(hidden=512, intermediate=1024, layers=layers, heads=4, kv_heads=2, head_dim=128, vocab=4096)
+    ir = build_decode_ir(256, cfg, argmax=True)
+    ex = DAGExecutor(partition(ir, is_hip_op_supported), backend,
+                     compile_fn=lambda sub: compile_subgraph(sub, persistent=False))
+    ex.load_weights(make_weights(ir, cfg, device="cuda"))
+    (hexec,) = ex.npu_executors.values()
+    assert hexec.use_graph and (len(hexec.program.steps) > 32) == (layers == 7)
+    x = {k: backend.allocate_buffer(v.cuda()) for k, v in decode_inputs(256, 100, cfg, seed=1).items()}
+    names = [o["name"] for o in ir["graph_outputs"]]
+    read = lambda y: [y[n].to_torch().clone() for n in names]
+    ids = x["input_ids"].native_handle
+    want = []
+    for tok in (3, 77, 1234):
+        ids.fill_(tok)
+        for _ in range(3):
+            y = read(ex.execute(x))
+        want.append(y)
+    assert len(hexec._graphs) == 1
+    print(f"[case] capture of {len(hexec.program.steps)} launches", flush=True)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        out = ex.execute(x)
+    for rep in range(2):
+        for tok, w in zip((3, 77, 1234), want):
+            ids.fill_(tok)
+            g.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(read(out), w)), (rep, tok)
+            assert all(torch.equal(a, b) for a, b in zip(read(ex.execute(x)), w)), (rep, tok)
